@@ -818,7 +818,6 @@ int atus_ctx_destroy(atus_ctx* c) {
   if (c->red_host) (void)hipHostFree(c->red_host);
   (void)hipFree(c->sob);
   (void)hipFree(c->lap);
-  (void)hipFree(c->grad);
   (void)hipFree(c->sob_st);
   (void)hipFree(c->sob_part);
   (void)hipFree(c->sob_log);
@@ -1665,72 +1664,88 @@ int sob_filter(atus_ctx* c, int comp, const double2* src, double2* out_sob, doub
   return ATUS_OK;
 }
 
-// the launches of one iteration up to the update: psi_sob, the Laplacian,
-// the Sobolev gradient and the projection products of every wave function
-// (Compute_Sobolev_Psi, Compute_Laplace, Compute_Sobolev_Gradient and the
-// dot products of Project_Sobolev_Gradient, CSOB_Base.h:251-367).  On 2D
-// and 3D grids the L2 gradient is formed inside the last-axis passes
-// (k_sob_gradfuse): the Laplacian's last inverse pass and the gradient
-// filter's first forward pass.
-int sob_body(atus_ctx* c) {
-  const int nw = c->ncomp, dim = c->dim;
-  const long long np = c->npts;
+// arguments of the Sobolev loop's kernels
+SobMix sob_mix_args(const atus_ctx* c) {
+  SobMix m{};
+  m.dim = c->dim;
+  for (int i = 0; i < c->ncomp; ++i) m.alpha[i] = c->sob_alpha[i];
+  for (int a = 0; a < 3; ++a) {
+    m.dk[a] = c->dk[a];
+    m.n[a] = c->n[a];
+  }
+  m.s = ft_factor(c->dim, c->dx) * ft_factor(c->dim, c->dk);
+  m.c = m.s * (double)c->npts;
+  return m;
+}
+
+// `count` iterations of a 2D/3D grid (sob.hpp):
+// the first spectra, then per iteration the middle axis, axis 0 twice and
+// the turn around the last axis
+int sob_loop(atus_ctx* c, int count, double eps) {
+  const int nw = c->ncomp, last = c->dim - 1, NL = c->n[last], N0 = c->n[0];
+  const long long np = c->npts, inner = c->inner_of(0);
   SobState* st = (SobState*)c->sob_st;
-  if (dim == 1) {
-    for (int i = 0; i < nw; ++i) ATUS_TRY(sob_filter(c, i, c->psi, c->sob, c->lap));
-    for (int i = 0; i < nw; ++i) {
-      hipLaunchKernelGGL(k_sob_grad_in, dim3(ew_blocks(np)), dim3(256), 0, c->stream, c->psi, c->lap, c->pot, c->grad,
-                         np, nw, i, c->gs[0 + i * nw], nw > 1 ? c->gs[1 + i * nw] : 0.0);
+  SobTurn ta{};
+  ta.pot = c->pot;
+  for (int i = 0; i < nw * nw; ++i) ta.gs[i] = c->gs[i];
+  ta.step = c->sob_step;
+  const SobMix mix = sob_mix_args(c);
+  ATUS_TRY(ensure_twiddles(c, N0));
+  ATUS_TRY(ensure_twiddles(c, NL));
+  const Limits lk = lim(c, ATUS_KFAM_KIN), lv = lim(c, ATUS_KFAM_VFUSE);
+  unsigned nbt = 0, nbm = 0;
+  HIP_TRY(launch_sob_turn(NL, nw, nullptr, nullptr, np, nullptr, ta, nullptr, nullptr, &nbt, lv, c->stream));
+  HIP_TRY(launch_sob_mix(N0, nw, nullptr, np, inner, nullptr, mix, nullptr, &nbm, lk, c->stream));
+  // partials of the turn, of the mix, and the mix's sums
+  const size_t need = 2 * (size_t)nw * ((size_t)nbt + nbm + 1);
+  if (c->sob_part_cap < need) {
+    HIP_TRY(hipStreamSynchronize(c->stream));
+    (void)hipFree(c->sob_part);
+    c->sob_part = nullptr;
+    c->sob_part_cap = 0;
+    if (hipMalloc(&c->sob_part, sizeof(double) * need) != hipSuccess) return fail(ATUS_ERR_NOMEM, "Sobolev partials");
+    c->sob_part_cap = need;
+  }
+  double* pt = c->sob_part;
+  double* pm = pt + 2 * (size_t)nw * nbt;
+  double* ps = pm + 2 * (size_t)nw * nbm;
+  SobFinish fin{pt, (int)nbt, nw, c->ar(), eps, 1, c->sob_log, 0};
+  ta.forward = 1;
+  HIP_TRY(launch_sob_turn(NL, nw, c->psi, c->sob, np, c->tw[NL], ta, st, pt, &nbt, lv, c->stream));
+  ta.update = 1;
+  for (int k = 0; k < count; ++k) {
+    if (c->dim == 3) ATUS_TRY(pass(c, 1, -1, c->sob, c->sob, 2 * nw, 1.0));
+    HIP_TRY(launch_sob_mix(N0, nw, c->sob, np, inner, c->tw[N0], mix, pm, &nbm, lk, c->stream));
+    // every workgroup of the pull sums the mix's partials: up to 1024 of
+    // them; more are summed once in between
+    const bool once = nbm > 1024;
+    for (int i = 0; once && i < nw; ++i) {
+      hipLaunchKernelGGL((k_reduce_final<2>), dim3(1), dim3(RED_THREADS), 0, c->stream, pm + 2 * (size_t)i * nbm,
+                         (int)nbm, ps + 2 * i);
       HIP_TRY(hipGetLastError());
-      ATUS_TRY(sob_filter(c, i, c->grad, c->grad, nullptr));
     }
-  } else {
-    const int last = dim - 1, NL = c->n[last], N0 = c->n[0];
-    SobArgs sa{};
-    sa.dim = dim;
-    for (int a = 0; a < 3; ++a) {
-      sa.dk[a] = c->dk[a];
-      sa.n[a] = c->n[a];
-    }
-    sa.scale = ft_factor(dim, c->dx) * ft_factor(dim, c->dk);
-    ATUS_TRY(ensure_twiddles(c, N0));
-    for (int i = 0; i < nw; ++i) {
-      // psi_sob complete; the Laplacian short of its last-axis inverse pass
-      const long long off = i * np;
-      sa.alpha = c->sob_alpha[i];
-      const double2* s = c->psi + off;
-      double2* w = c->sob + off;
-      for (int a = last; a >= 1; --a) {
-        ATUS_TRY(pass(c, a, -1, s, w, 1, 1.0));
-        s = w;
-      }
-      HIP_TRY(launch_sobf(N0, c->rm[ATUS_KFAM_KIN], false, s, w, c->lap + off, np, 1, c->inner_of(0), c->tw[N0], sa,
-                          lim(c, ATUS_KFAM_KIN), c->stream));
-      for (int a = 1; a <= last; ++a) ATUS_TRY(pass(c, a, +1, w, w, 1, 1.0));
-      for (int a = 1; a < last; ++a) ATUS_TRY(pass(c, a, +1, c->lap + off, c->lap + off, 1, 1.0));
-    }
-    for (int i = 0; i < nw; ++i) {
-      const long long off = i * np;
-      sa.alpha = c->sob_alpha[i];
-      double2* w = c->grad + off;
-      HIP_TRY(launch_sob_gradfuse(NL, c->rm[ATUS_KFAM_VFUSE], nw, c->lap, c->psi, c->pot, c->grad, np, i,
-                                  c->gs[0 + i * nw], nw > 1 ? c->gs[1 + i * nw] : 0.0, c->tw[NL], lim(c, ATUS_KFAM_VFUSE),
-                                  c->stream));
-      for (int a = last - 1; a >= 1; --a) ATUS_TRY(pass(c, a, -1, w, w, 1, 1.0));
-      HIP_TRY(launch_sobf(N0, c->rm[ATUS_KFAM_KIN], false, w, w, nullptr, np, 1, c->inner_of(0), c->tw[N0], sa,
-                          lim(c, ATUS_KFAM_KIN), c->stream));
-      for (int a = 1; a <= last; ++a) ATUS_TRY(pass(c, a, +1, w, w, 1, 1.0));
-    }
+    HIP_TRY(launch_sob_pull(N0, nw, c->sob, np, inner, c->tw[N0], once ? ps : pm, once ? 1 : (int)nbm, st, fin, lk,
+                            c->stream));
+    if (c->dim == 3) ATUS_TRY(pass(c, 1, +1, c->sob, c->sob, nw, 1.0));
+    ta.forward = k + 1 < count;
+    HIP_TRY(launch_sob_turn(NL, nw, c->psi, c->sob, np, c->tw[NL], ta, st, pt, &nbt, lv, c->stream));
+    fin.init = 0;
+    fin.slot = k;
   }
-  for (int i = 0; i < nw; ++i) {
-    RedProj fp{c->psi + i * np, c->grad + i * np, c->sob + i * np};
-    const unsigned nb = red_blocks(np);
-    hipLaunchKernelGGL((k_reduce<RedProj>), dim3(nb), dim3(RED_THREADS), 0, c->stream, fp, np, c->red_part);
-    HIP_TRY(hipGetLastError());
-    hipLaunchKernelGGL((k_reduce_final<2>), dim3(1), dim3(RED_THREADS), 0, c->stream, c->red_part, (int)nb,
-                       &st->proj[i][0]);
-    HIP_TRY(hipGetLastError());
-  }
+  hipLaunchKernelGGL(k_sob_finish, dim3(1), dim3(RED_THREADS), 0, c->stream, st, fin);
+  HIP_TRY(hipGetLastError());
+  return ATUS_OK;
+}
+
+// `count` iterations of a 1D grid in one launch
+int sob_loop_line(atus_ctx* c, int count, double eps) {
+  SobTurn ta{};
+  ta.pot = c->pot;
+  for (int i = 0; i < c->ncomp * c->ncomp; ++i) ta.gs[i] = c->gs[i];
+  ta.step = c->sob_step;
+  ATUS_TRY(ensure_twiddles(c, c->n[0]));
+  HIP_TRY(launch_sob_line(c->n[0], c->ncomp, c->psi, c->tw[c->n[0]], ta, sob_mix_args(c), c->ar(), eps, count,
+                          (SobState*)c->sob_st, c->sob_log, lim(c, ATUS_KFAM_KIN), c->stream));
   return ATUS_OK;
 }
 
@@ -1765,11 +1780,9 @@ int atus_sob_setup(atus_ctx* c, const double* alpha_iso, double stepsize) {
   for (int i = 0; i < c->ncomp; ++i) c->sob_alpha[i] = alpha_iso[i];
   c->sob_step = stepsize;
   const size_t bytes = sizeof(double2) * c->npts * c->ncomp;
-  if (!c->sob && hipMalloc(&c->sob, bytes) != hipSuccess) return fail(ATUS_ERR_NOMEM, "Sobolev buffers");
+  if (!c->sob && hipMalloc(&c->sob, 2 * bytes) != hipSuccess) return fail(ATUS_ERR_NOMEM, "Sobolev buffers");
   if (!c->lap && hipMalloc(&c->lap, bytes) != hipSuccess) return fail(ATUS_ERR_NOMEM, "Sobolev buffers");
-  if (!c->grad && hipMalloc(&c->grad, bytes) != hipSuccess) return fail(ATUS_ERR_NOMEM, "Sobolev buffers");
   if ((!c->sob_st && hipMalloc(&c->sob_st, sizeof(SobState)) != hipSuccess) ||
-      (!c->sob_part && hipMalloc(&c->sob_part, sizeof(double) * 2 * RED_MAX_BLOCKS * 2) != hipSuccess) ||
       (!c->sob_log && hipMalloc(&c->sob_log, sizeof(double) * SOB_MAX_CHUNK * SOB_LOG_VALS) != hipSuccess))
     return fail(ATUS_ERR_NOMEM, "Sobolev loop state");
   c->sob_ready = true;
@@ -1796,36 +1809,9 @@ int atus_sob_iterate(atus_ctx* c, int count, double eps, int* performed, double*
   if (!c->sob_ready) return fail(ATUS_ERR_STATE, "call atus_sob_setup first");
   if (count < 1 || count > SOB_MAX_CHUNK)
     return fail(ATUS_ERR_ARG, "count must be 1.." + std::to_string(SOB_MAX_CHUNK));
-  const int nw = c->ncomp;
-  const long long np = c->npts;
-  const unsigned nb = red_blocks(np);
-  SobState* st = (SobState*)c->sob_st;
-  auto finalize = [&](int init, int slot) -> int {
-    hipLaunchKernelGGL(k_sob_finalize, dim3(1), dim3(RED_THREADS), 0, c->stream, st, c->sob_part, (int)nb, nw, c->ar(),
-                       eps, init, c->sob_log, slot);
-    HIP_TRY(hipGetLastError());
-    return ATUS_OK;
-  };
-  // N of the current psi, the renormalisation of the first iteration
-  for (int i = 0; i < nw; ++i) {
-    hipLaunchKernelGGL(k_sob_update_dev, dim3(nb), dim3(RED_THREADS), 0, c->stream, c->psi + i * np,
-                       (const double2*)nullptr, (const double2*)nullptr, np, 0.0, (const SobState*)st, i, 1,
-                       c->sob_part + (size_t)i * nb * 2);
-    HIP_TRY(hipGetLastError());
-  }
-  ATUS_TRY(finalize(1, 0));
-  for (int k = 0; k < count; ++k) {
-    ATUS_TRY(sob_body(c));
-    for (int i = 0; i < nw; ++i) {
-      hipLaunchKernelGGL(k_sob_update_dev, dim3(nb), dim3(RED_THREADS), 0, c->stream, c->psi + i * np,
-                         (const double2*)c->grad + i * np, (const double2*)c->sob + i * np, np, c->sob_step,
-                         (const SobState*)st, i, 0, c->sob_part + (size_t)i * nb * 2);
-      HIP_TRY(hipGetLastError());
-    }
-    ATUS_TRY(finalize(0, k));
-  }
+  ATUS_TRY(c->dim == 1 ? sob_loop_line(c, count, eps) : sob_loop(c, count, eps));
   SobState h;
-  HIP_TRY(hipMemcpyAsync(&h, st, sizeof(SobState), hipMemcpyDeviceToHost, c->stream));
+  HIP_TRY(hipMemcpyAsync(&h, c->sob_st, sizeof(SobState), hipMemcpyDeviceToHost, c->stream));
   std::vector<double> lg;
   if (log) {
     lg.resize((size_t)count * SOB_LOG_VALS);

@@ -102,11 +102,14 @@ struct atus_ctx {
   bool sob_ready = false;
   double sob_alpha[2] = {0, 0};
   double sob_step = 0;
-  double2 *sob = nullptr, *lap = nullptr, *grad = nullptr;
-  // the device-side loop: its state (atus::SobState), the update partials
-  // [2][RED_MAX_BLOCKS][2] and the per-iteration log [SOB_MAX_CHUNK][4]
+  // the iteration's spectra [2 ncomp][npts] (k_sob_turn), the Laplacian of
+  // the chemical potential
+  double2 *sob = nullptr, *lap = nullptr;
+  // the device-side loop: its state (atus::SobState), the passes' partial
+  // sums and the per-iteration log [SOB_MAX_CHUNK][4]
   void* sob_st = nullptr;
   double* sob_part = nullptr;
+  size_t sob_part_cap = 0;
   double* sob_log = nullptr;
 
   bool timing = false;

@@ -28,7 +28,7 @@ static int pencil_lds_elems(int N, int P, bool contig, long long T) {
 }
 
 PassCfg make_pass_cfg(int N, int rm, long long inner, long long outer, int ycount, size_t max_lds, int ntables,
-                      int max_threads, long long table_elems) {
+                      int max_threads, long long table_elems, int min_threads) {
   PassCfg c{};
   const int P = threads_per_pencil(N, rm);
   const bool contig = inner == 1;
@@ -37,7 +37,7 @@ PassCfg make_pass_cfg(int N, int rm, long long inner, long long outer, int ycoun
                                          : 0;
   long long T = max_threads / P;
   if (T < 1) T = 1;
-  if (!contig && T > inner) T = inner;
+  if (!contig && T > inner) T = inner * P >= min_threads ? inner : min_threads / P;
   auto pencil_bytes = [&](long long t) { return (size_t)pencil_lds_elems(N, P, contig, t) * sizeof(double2); };
   while (T > 1 && (size_t)T * pencil_bytes(T) + table_bytes > max_lds) T >>= 1;
   if (inner == 1) {

@@ -7,6 +7,11 @@
 
 namespace atus {
 
+struct SobTurn;
+struct SobMix;
+struct SobFinish;
+struct SobState;
+
 // workgroup shape of one axis pass: T pencils of P = N/min(16,N) threads
 struct PassCfg {
   dim3 grid;
@@ -30,18 +35,20 @@ struct Limits {
 // [N][inner]; ycount = gridDim.y (components)
 // ntables: lookup tables of length N the kernel stages in LDS (N <= 1024);
 // table_elems >= 0 gives the LDS table elements exactly instead
+// min_threads: strided passes of fewer columns than that many threads hold
+// take workgroups of that size all the same (their spare columns are invalid)
 PassCfg make_pass_cfg(int N, int rm, long long inner, long long outer, int ycount, size_t max_lds,
-                      int ntables = 1, int max_threads = 256, long long table_elems = -1);
+                      int ntables = 1, int max_threads = 256, long long table_elems = -1, int min_threads = 0);
 // the same within Limits (max_threads: the kernel's launch bounds)
 inline PassCfg make_pass_cfg(int N, int rm, long long inner, long long outer, int ycount, const Limits& lim,
-                             int ntables = 1, int max_threads = 256, long long table_elems = -1) {
+                             int ntables = 1, int max_threads = 256, long long table_elems = -1, int min_threads = 0) {
   int t = max_threads;
   if (lim.threads > 0) {
     const int P = threads_per_pencil(N, rm);
     t = lim.threads < max_threads ? lim.threads : max_threads;
     if (t < P) t = P < max_threads ? P : max_threads;
   }
-  return make_pass_cfg(N, rm, inner, outer, ycount, lim.lds, ntables, t, table_elems);
+  return make_pass_cfg(N, rm, inner, outer, ycount, lim.lds, ntables, t, table_elems, min_threads);
 }
 
 bool supported_len(int N);  // power of two in [2, 4096]
@@ -117,12 +124,21 @@ hipError_t launch_sobf(int N, int rm, bool contig, const double2* src, double2* 
                        long long comp_stride, int ncomp, long long inner, const double2* tw, const SobArgs& sa,
                        const Limits& max_lds, hipStream_t s);
 
-// the Sobolev iteration's L2 gradient of component `comp` fused into the
-// last-axis inverse (Laplacian) and forward (gradient filter) passes of a
-// 2D/3D grid of nw (1 or 2) wave functions
-hipError_t launch_sob_gradfuse(int N, int rm, int nw, const double2* lap, const double2* psi, const double* pot,
-                               double2* out, long long npts, int comp, double g0, double g1, const double2* tw,
-                               const Limits& max_lds, hipStream_t s);
+// the passes of a Sobolev iteration on a 2D/3D grid of nw (1 or 2) wave
+// functions (sob.hpp); partials NULL: only *nblocks,
+// the workgroups per component, is set
+hipError_t launch_sob_turn(int N, int nw, double2* psi, double2* spec, long long npts, const double2* tw,
+                           const SobTurn& a, const SobState* st, double* partials, unsigned* nblocks,
+                           const Limits& lim, hipStream_t s);
+hipError_t launch_sob_mix(int N, int nw, double2* spec, long long npts, long long inner, const double2* tw,
+                          const SobMix& sa, double* partials, unsigned* nblocks, const Limits& lim, hipStream_t s);
+hipError_t launch_sob_pull(int N, int nw, double2* spec, long long npts, long long inner, const double2* tw,
+                           const double* partials, int nb, SobState* st, const SobFinish& fin, const Limits& lim,
+                           hipStream_t s);
+// up to `count` iterations of a 1D grid in one launch
+hipError_t launch_sob_line(int N, int nw, double2* psi, const double2* tw, const SobTurn& a, const SobMix& sa,
+                           double ar, double eps, int count, SobState* st, double* log, const Limits& lim,
+                           hipStream_t s);
 
 // pointwise V step on all points (unfused path)
 hipError_t launch_point(int vk, int nc, double2* psi, const Grid& gr, const VArgs& va, hipStream_t s);

@@ -249,7 +249,7 @@ int atus_run_block_profiled(atus_ctx *ctx, const atus_step_params *sp, int Nk, d
                             double *grid);
 
 /* tuning: values per thread (8 or 16) of the FFT kernels of one kernel
- * family (ATUS_KFAM_*; the Sobolev filter follows ATUS_KFAM_KIN).  16 halves
+ * family (ATUS_KFAM_*; the Sobolev minimiser's iteration takes 8 always).  16 halves
  * the LDS exchanges, 8 halves the registers per thread.  Defaults: 16 for
  * the contiguous passes and the kinetic step, 8 for the strided passes and
  * the fused V pass. */
