@@ -37,7 +37,10 @@ PassCfg make_pass_cfg(int N, int rm, long long inner, long long outer, int ycoun
                                          : 0;
   long long T = max_threads / P;
   if (T < 1) T = 1;
-  if (!contig && T > inner) T = inner * P >= min_threads ? inner : min_threads / P;
+  if (!contig && T > inner) {
+    const long long q = P < min_threads ? min_threads / P : 1;
+    T = (inner + q - 1) / q * q;
+  }
   auto pencil_bytes = [&](long long t) { return (size_t)pencil_lds_elems(N, P, contig, t) * sizeof(double2); };
   while (T > 1 && (size_t)T * pencil_bytes(T) + table_bytes > max_lds) T >>= 1;
   if (inner == 1) {
@@ -128,7 +131,7 @@ static hipError_t rabi_nr(int axis, const double2* src, long long seg, int nseg,
   PassCfg c;
   if (axis == 2) c = make_pass_cfg(N, RM, 1, (long long)rb.n[0] * rb.n[1], nseg, lim);
   else if (axis == 1) c = make_pass_cfg(N, RM, rb.len[2], rb.n[0], nseg, lim);
-  else c = make_pass_cfg(N, RM, (long long)rb.len[1] * rb.len[2], 1, nseg, lim);
+  else c = make_pass_cfg(N, RM, (long long)rb.len[1] * rb.len[2], 1, nseg, lim, 1, 256, -1, 64);
   if (c.block.x == 0 || c.block.x > 256 || c.grid.x == 0) return hipErrorInvalidConfiguration;
   static bool ok[3] = {false, false, false};
   hipError_t e;
