@@ -83,6 +83,16 @@ namespace {
 // the family's tuned threads per workgroup (atus_tune_threads)
 Limits lim(const atus_ctx* c, int fam) { return Limits{c->max_lds, c->wg[fam]}; }
 
+// values per thread of kernel family fam: the tuned choice, else 8 for the
+// strided passes and the V pass (which spills at 16), and 16, half the
+// exchanges, for the contiguous passes and the kinetic step of a state large
+// enough to give every CU two workgroups of 256 threads all the same
+int vals(const atus_ctx* c, int fam) {
+  if (c->rm[fam]) return c->rm[fam];
+  if (fam == ATUS_KFAM_PASS_STRIDED || fam == ATUS_KFAM_VFUSE) return 8;
+  return c->npts * c->ncomp >= 2LL * CU_COUNT * 256 * 16 ? 16 : 8;
+}
+
 int check_ctx(atus_ctx* c) {
   if (!c) return fail(ATUS_ERR_ARG, "null context");
   return hipSetDevice(c->device) == hipSuccess ? ATUS_OK : fail(ATUS_ERR_HIP, "hipSetDevice failed");
@@ -272,7 +282,7 @@ int pass(atus_ctx* c, int a, int dir, const double2* src, double2* dst, int ncom
   const long long inner = c->inner_of(a), outer = c->outer_of(a);
   const int fam = inner == 1 ? ATUS_KFAM_PASS_CONTIG : ATUS_KFAM_PASS_STRIDED;
   ProfScope ps(c, fam);
-  HIP_TRY(launch_pass(N, c->rm[fam], inner == 1, dir, src, dst, cs ? cs : c->npts, ncomp, inner, outer, c->tw[N], scale,
+  HIP_TRY(launch_pass(N, vals(c, fam), inner == 1, dir, src, dst, cs ? cs : c->npts, ncomp, inner, outer, c->tw[N], scale,
                       lim(c, fam), c->stream));
   return ATUS_OK;
 }
@@ -287,7 +297,7 @@ int pass_slab(atus_ctx* c, int a, int dir, int s0, int S, hipStream_t st) {
   const int fam = inner == 1 ? ATUS_KFAM_PASS_CONTIG : ATUS_KFAM_PASS_STRIDED;
   double2* p = c->psi + (long long)s0 * plane;
   ProfScope ps(c, fam, (double)S / c->n[0], st);
-  HIP_TRY(launch_pass(N, c->rm[fam], inner == 1, dir, p, p, c->npts, c->ncomp, inner, outer, c->tw[N], 1.0, lim(c, fam),
+  HIP_TRY(launch_pass(N, vals(c, fam), inner == 1, dir, p, p, c->npts, c->ncomp, inner, outer, c->tw[N], 1.0, lim(c, fam),
                       st));
   return ATUS_OK;
 }
@@ -303,7 +313,7 @@ int vfuse_slab(atus_ctx* c, int vk, const VArgs& va, int s0, int S, hipStream_t 
   VArgs vs = va;
   if (vs.pot) vs.pot += (long long)s0 * plane;
   ProfScope ps(c, ATUS_KFAM_VFUSE, (double)S / c->n[0], st);
-  HIP_TRY(launch_vfuse(NL, c->rm[ATUS_KFAM_VFUSE], vk, c->ncomp, c->psi + (long long)s0 * plane, c->npts,
+  HIP_TRY(launch_vfuse(NL, vals(c, ATUS_KFAM_VFUSE), vk, c->ncomp, c->psi + (long long)s0 * plane, c->npts,
                        (long long)S * c->n[1], c->tw[NL], vs, c->n[1], c->n[0] - 2 * s0, c->dx[0], lim(c, ATUS_KFAM_VFUSE),
                        st, edge ? axis_tabs(c, 2).e0 : nullptr, edge));
   return ATUS_OK;
@@ -318,7 +328,7 @@ int kin_y_slab(atus_ctx* c, const VArgs& va, int s0, int S, hipStream_t st) {
   ATUS_TRY(ensure_twiddles(c, N));
   const long long plane = (long long)c->n[1] * c->n[2];
   ProfScope ps(c, ATUS_KFAM_PASS_STRIDED, (double)S / c->n[0], st);
-  HIP_TRY(launch_kin(N, c->rm[ATUS_KFAM_PASS_STRIDED], false, V_NONE, 1, c->psi + (long long)s0 * plane, c->npts,
+  HIP_TRY(launch_kin(N, vals(c, ATUS_KFAM_PASS_STRIDED), false, V_NONE, 1, c->psi + (long long)s0 * plane, c->npts,
                      c->ncomp, c->n[2], c->tw[N], axis_tabs(c, 1), va, c->dx[0], lim(c, ATUS_KFAM_PASS_STRIDED), st,
                      S));
   return ATUS_OK;
@@ -329,7 +339,7 @@ int kin_y_slab(atus_ctx* c, const VArgs& va, int s0, int S, hipStream_t st) {
 int fs_col(atus_ctx* c, int mode, double2* p, int ycount, long long cs, int vk, int nc, bool batch, const VArgs& va,
            double scale) {
   ProfScope ps(c, mode == FS_STEP ? ATUS_KFAM_VFUSE : ATUS_KFAM_PASS_STRIDED);
-  HIP_TRY(launch_fs_col(c->fs_n1, c->rm[mode == FS_STEP ? ATUS_KFAM_VFUSE : ATUS_KFAM_PASS_STRIDED], mode, vk, nc, batch,
+  HIP_TRY(launch_fs_col(c->fs_n1, vals(c, mode == FS_STEP ? ATUS_KFAM_VFUSE : ATUS_KFAM_PASS_STRIDED), mode, vk, nc, batch,
                         p, cs, ycount, c->fs_n2, c->tw[c->fs_n1], c->tw[(int)c->npts], va, c->dx[0], scale,
                         lim(c, mode == FS_STEP ? ATUS_KFAM_VFUSE : ATUS_KFAM_PASS_STRIDED), c->stream));
   return ATUS_OK;
@@ -338,7 +348,7 @@ int fs_col(atus_ctx* c, int mode, double2* p, int ycount, long long cs, int vk, 
 // four-step row pass of ncomp components: kinetic phase of slot f
 int fs_row_kin(atus_ctx* c, int f, const VArgs& va) {
   ProfScope ps(c, ATUS_KFAM_KIN);
-  HIP_TRY(launch_kin(c->fs_n2, c->rm[ATUS_KFAM_KIN], true, V_NONE, 1, c->psi, c->npts, c->ncomp, 1, c->tw[c->fs_n2],
+  HIP_TRY(launch_kin(c->fs_n2, vals(c, ATUS_KFAM_KIN), true, V_NONE, 1, c->psi, c->npts, c->ncomp, 1, c->tw[c->fs_n2],
                      kin_tabs(c, f), va, c->dx[0], lim(c, ATUS_KFAM_KIN), c->stream, c->fs_n1));
   return ATUS_OK;
 }
@@ -377,7 +387,7 @@ int full_ft(atus_ctx* c, int dir, const double2* src, double2* dst, int ncomp, l
       ATUS_TRY(fs_col(c, FS_ENTER, dst, ncomp, s_, V_NONE, 1, false, none, 1.0));
       {
         ProfScope ps(c, ATUS_KFAM_PASS_CONTIG);
-        HIP_TRY(launch_pass(c->fs_n2, c->rm[ATUS_KFAM_PASS_CONTIG], true, -1, dst, dst, s_, ncomp, 1, c->fs_n1,
+        HIP_TRY(launch_pass(c->fs_n2, vals(c, ATUS_KFAM_PASS_CONTIG), true, -1, dst, dst, s_, ncomp, 1, c->fs_n1,
                             c->tw[c->fs_n2], 1.0, lim(c, ATUS_KFAM_PASS_CONTIG), c->stream));
       }
       ATUS_TRY(transpose(c, dst, t, c->fs_n1, c->fs_n2, ncomp, s_, scale));
@@ -387,7 +397,7 @@ int full_ft(atus_ctx* c, int dir, const double2* src, double2* dst, int ncomp, l
       ATUS_TRY(transpose(c, src, t, c->fs_n2, c->fs_n1, ncomp, s_, scale));
       {
         ProfScope ps(c, ATUS_KFAM_PASS_CONTIG);
-        HIP_TRY(launch_pass(c->fs_n2, c->rm[ATUS_KFAM_PASS_CONTIG], true, +1, t, t, s_, ncomp, 1, c->fs_n1,
+        HIP_TRY(launch_pass(c->fs_n2, vals(c, ATUS_KFAM_PASS_CONTIG), true, +1, t, t, s_, ncomp, 1, c->fs_n1,
                             c->tw[c->fs_n2], 1.0, lim(c, ATUS_KFAM_PASS_CONTIG), c->stream));
       }
       ATUS_TRY(fs_col(c, FS_EXIT, t, ncomp, s_, V_NONE, 1, false, none, 1.0));
@@ -420,7 +430,7 @@ int kinetic_unfused(atus_ctx* c, int f) {
   VArgs va{};
   {
     ProfScope ps(c, ATUS_KFAM_KIN);
-    HIP_TRY(launch_kin(N0, c->rm[ATUS_KFAM_KIN], c->dim == 1, V_NONE, 1, c->psi, c->npts, c->ncomp, c->inner_of(0), c->tw[N0],
+    HIP_TRY(launch_kin(N0, vals(c, ATUS_KFAM_KIN), c->dim == 1, V_NONE, 1, c->psi, c->npts, c->ncomp, c->inner_of(0), c->tw[N0],
                        kin_tabs(c, f), va, c->dx[0], lim(c, ATUS_KFAM_KIN), c->stream));
   }
   for (int a = 1; a < c->dim; ++a) ATUS_TRY(pass(c, a, +1, c->psi, c->psi, c->ncomp, 1.0));
@@ -599,7 +609,7 @@ int ensure_rabi_box(atus_ctx* c, const RabiReduction& rr, int nseg) {
   unsigned nb = 0;
   rb.len[1] = rr.box.len[1];
   rb.len[2] = rr.box.len[2];
-  HIP_TRY(launch_rabi_box(0, c->rm[ATUS_KFAM_PASS_STRIDED], nullptr, 0, nseg, nullptr, nullptr, c->tw[c->n[0]], rb,
+  HIP_TRY(launch_rabi_box(0, vals(c, ATUS_KFAM_PASS_STRIDED), nullptr, 0, nseg, nullptr, nullptr, c->tw[c->n[0]], rb,
                           lim(c, ATUS_KFAM_PASS_STRIDED), nullptr, &nb, c->stream));
   return ensure_sred(c, (size_t)nseg * nb * RED_MAX_NV, nseg);
 }
@@ -626,14 +636,14 @@ int rabi_box3(atus_ctx* c, const double2* src, long long seg, int nseg, const Ra
   double2* zb = c->rbuf;
   double2* yb = c->rbuf + (size_t)nseg * c->n[0] * c->n[1] * rb.len[2];
   unsigned nb = 0;
-  HIP_TRY(launch_rabi_box(2, c->rm[ATUS_KFAM_PASS_CONTIG], src, seg, nseg, zb, yb, c->tw[c->n[2]], rb,
+  HIP_TRY(launch_rabi_box(2, vals(c, ATUS_KFAM_PASS_CONTIG), src, seg, nseg, zb, yb, c->tw[c->n[2]], rb,
                           lim(c, ATUS_KFAM_PASS_CONTIG), nullptr, nullptr, c->stream));
-  HIP_TRY(launch_rabi_box(1, c->rm[ATUS_KFAM_PASS_STRIDED], src, seg, nseg, zb, yb, c->tw[c->n[1]], rb,
+  HIP_TRY(launch_rabi_box(1, vals(c, ATUS_KFAM_PASS_STRIDED), src, seg, nseg, zb, yb, c->tw[c->n[1]], rb,
                           lim(c, ATUS_KFAM_PASS_STRIDED), nullptr, nullptr, c->stream));
-  HIP_TRY(launch_rabi_box(0, c->rm[ATUS_KFAM_PASS_STRIDED], src, seg, nseg, zb, yb, c->tw[c->n[0]], rb,
+  HIP_TRY(launch_rabi_box(0, vals(c, ATUS_KFAM_PASS_STRIDED), src, seg, nseg, zb, yb, c->tw[c->n[0]], rb,
                           lim(c, ATUS_KFAM_PASS_STRIDED), nullptr, &nb, c->stream));
   if (c->sred_cap < (size_t)nseg * nb * RED_MAX_NV) return fail(ATUS_ERR_STATE, "reduction buffers not sized");
-  HIP_TRY(launch_rabi_box(0, c->rm[ATUS_KFAM_PASS_STRIDED], src, seg, nseg, zb, yb, c->tw[c->n[0]], rb,
+  HIP_TRY(launch_rabi_box(0, vals(c, ATUS_KFAM_PASS_STRIDED), src, seg, nseg, zb, yb, c->tw[c->n[0]], rb,
                           lim(c, ATUS_KFAM_PASS_STRIDED), c->sred_part, &nb, c->stream));
   hipLaunchKernelGGL((k_reduce_seg_final<RED_MAX_NV>), dim3((unsigned)nseg), dim3(RED_THREADS), 0, c->stream,
                      c->sred_part, (int)nb, res);
@@ -1094,7 +1104,7 @@ int single_block_slabs(atus_ctx* c, int vk, const VArgs& base, int Nk, double dt
     ProfScope ps(c, ATUS_KFAM_KIN);
     const bool rev = comp0_last && kt.f0 == nullptr && c->ncomp > 1;
     double2* base = rev ? c->psi + (long long)(c->ncomp - 1) * c->npts : c->psi;
-    HIP_TRY(launch_kin(N0, c->rm[ATUS_KFAM_KIN], false, V_NONE, 1, base, rev ? -c->npts : c->npts, c->ncomp, inner0,
+    HIP_TRY(launch_kin(N0, vals(c, ATUS_KFAM_KIN), false, V_NONE, 1, base, rev ? -c->npts : c->npts, c->ncomp, inner0,
                        c->tw[N0], kt, va, c->dx[0], lim(c, ATUS_KFAM_KIN), c->stream));
     return ATUS_OK;
   };
@@ -1234,7 +1244,7 @@ int single_block(atus_ctx* c, int vk, const VArgs& base, int Nk, double dt, doub
   double tt = *t;
   auto kin2d = [&](const KinTabs& kt, const VArgs& va) -> int {
     ProfScope ps(c, ATUS_KFAM_KIN);
-    HIP_TRY(launch_kin(N0, c->rm[ATUS_KFAM_KIN], false, V_NONE, 1, c->psi, c->npts, c->ncomp, inner0, c->tw[N0], kt,
+    HIP_TRY(launch_kin(N0, vals(c, ATUS_KFAM_KIN), false, V_NONE, 1, c->psi, c->npts, c->ncomp, inner0, c->tw[N0], kt,
                        va, c->dx[0], lim(c, ATUS_KFAM_KIN), c->stream));
     return ATUS_OK;
   };
@@ -1265,13 +1275,13 @@ int single_block(atus_ctx* c, int vk, const VArgs& base, int Nk, double dt, doub
       ATUS_TRY(fs_row_kin(c, f, va));
     } else if (c->dim == 1) {
       ProfScope ps(c, ATUS_KFAM_KIN);
-      HIP_TRY(launch_kin(N0, c->rm[ATUS_KFAM_KIN], true, vk, c->ncomp, c->psi, c->npts, c->ncomp, 1, c->tw[N0], kin_tabs(c, f), va,
+      HIP_TRY(launch_kin(N0, vals(c, ATUS_KFAM_KIN), true, vk, c->ncomp, c->psi, c->npts, c->ncomp, 1, c->tw[N0], kin_tabs(c, f), va,
                          c->dx[0], lim(c, ATUS_KFAM_KIN), c->stream));
     } else {
       const int edge = (m == 1 ? 1 : 0) | (m == Nk ? 2 : 0);
       {
         ProfScope ps(c, ATUS_KFAM_VFUSE);
-        HIP_TRY(launch_vfuse(NL, c->rm[ATUS_KFAM_VFUSE], vk, c->ncomp, c->psi, c->npts, c->npts / NL, c->tw[NL], va, 1,
+        HIP_TRY(launch_vfuse(NL, vals(c, ATUS_KFAM_VFUSE), vk, c->ncomp, c->psi, c->npts, c->npts / NL, c->tw[NL], va, 1,
                              c->n[0], c->dx[0], lim(c, ATUS_KFAM_VFUSE), c->stream, edge ? axis_tabs(c, 1).e0 : nullptr,
                              edge));
       }
@@ -1300,7 +1310,7 @@ int batch_block(atus_ctx* c, int vk, const VArgs& base, int Nk, double dt, doubl
   double tt = *t;
   auto kin = [&](const KinTabs& kt, const VArgs& va) -> int {
     ProfScope ps(c, ATUS_KFAM_KIN);
-    HIP_TRY(launch_kin(N0, c->rm[ATUS_KFAM_KIN], false, V_NONE, 1, c->psi, c->npts, c->ncomp, inner0, c->tw[N0], kt,
+    HIP_TRY(launch_kin(N0, vals(c, ATUS_KFAM_KIN), false, V_NONE, 1, c->psi, c->npts, c->ncomp, inner0, c->tw[N0], kt,
                        va, c->dx[0], lim(c, ATUS_KFAM_KIN), c->stream));
     return ATUS_OK;
   };
@@ -1327,7 +1337,7 @@ int batch_block(atus_ctx* c, int vk, const VArgs& base, int Nk, double dt, doubl
       ATUS_TRY(fs_row_kin(c, f, va));
     } else if (c->dim == 1) {
       ProfScope ps(c, ATUS_KFAM_KIN);
-      HIP_TRY(launch_vstep_batch(N0, c->rm[ATUS_KFAM_KIN], true, vk, c->psi, c->npts, B, c->tw[N0], kin_tabs(c, f), va,
+      HIP_TRY(launch_vstep_batch(N0, vals(c, ATUS_KFAM_KIN), true, vk, c->psi, c->npts, B, c->tw[N0], kin_tabs(c, f), va,
                                  1, N0, c->dx[0], lim(c, ATUS_KFAM_KIN), c->stream));
     } else {
       const bool first = m == 1, last = m == Nk;
@@ -1339,7 +1349,7 @@ int batch_block(atus_ctx* c, int vk, const VArgs& base, int Nk, double dt, doubl
       }
       {
         ProfScope ps(c, ATUS_KFAM_VFUSE);
-        HIP_TRY(launch_vstep_batch(NL, c->rm[ATUS_KFAM_VFUSE], false, vk, c->psi, c->npts,
+        HIP_TRY(launch_vstep_batch(NL, vals(c, ATUS_KFAM_VFUSE), false, vk, c->psi, c->npts,
                                    (long long)B * base.pencils_per_run, c->tw[NL], kin_tabs(c, f), va, ppx, c->n[0],
                                    c->dx[0], lim(c, ATUS_KFAM_VFUSE), c->stream,
                                    edge ? axis_tabs(c, c->dim - 1).e0 : nullptr, edge));
@@ -1655,7 +1665,7 @@ int sob_filter(atus_ctx* c, int comp, const double2* src, double2* out_sob, doub
   }
   const int N0 = c->n[0];
   ATUS_TRY(ensure_twiddles(c, N0));
-  HIP_TRY(launch_sobf(N0, c->rm[ATUS_KFAM_KIN], c->dim == 1, s, w, out_lap ? out_lap + off : nullptr, c->npts, 1, c->inner_of(0),
+  HIP_TRY(launch_sobf(N0, vals(c, ATUS_KFAM_KIN), c->dim == 1, s, w, out_lap ? out_lap + off : nullptr, c->npts, 1, c->inner_of(0),
                       c->tw[N0], sa, lim(c, ATUS_KFAM_KIN), c->stream));
   for (int a = 1; a < c->dim; ++a) {
     ATUS_TRY(pass(c, a, +1, w, w, 1, 1.0));

@@ -116,12 +116,12 @@ struct atus_ctx {
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   double last_ms = 0;
 
-  // values per thread of the FFT kernels, per kernel family (ATUS_KFAM_*);
-  // defaults: what the autotuner picks at 256^3 (8 for the strided passes
-  // and for the register-heavy V pass, which spills at 16)
-  int rm[ATUS_NKFAM] = {16, 8, 16, 8, 16};
+  // values per thread of the FFT kernels, per kernel family (ATUS_KFAM_*):
+  // 8 or 16 as tuned, 0: by the state's size (vals in atus_abi.hip)
+  int rm[ATUS_NKFAM] = {0, 0, 0, 0, 0};
   // threads per workgroup at most, per kernel family (0: as many as the
-  // kernel's launch bounds allow); sets the pencils per workgroup
+  // kernel's launch bounds allow and the device's CUs leave); sets the
+  // pencils per workgroup
   int wg[ATUS_NKFAM] = {0, 0, 0, 0, 0};
   // 3D blocks: the y and z passes between two kinetic steps run slab by
   // slab of this many x-planes, alternate slabs on two streams (0: over the

@@ -23,9 +23,12 @@ struct PassCfg {
 // values per thread R = min(rm, N); threads per pencil P = N / R
 inline int threads_per_pencil(int N, int rm) { return N / (N < rm ? N : rm); }
 
+constexpr int CU_COUNT = 256;  // compute units of MI355X
+
 // what a launch may use: LDS bytes per workgroup, and threads per
-// workgroup at most (0: as many as the kernel's launch bounds allow; the
-// pencils per workgroup follow as threads / P, at least one pencil)
+// workgroup at most (the pencils per workgroup follow as threads / P, at
+// least one pencil).  0: as many as the kernel's launch bounds allow, halved
+// down to one wavefront while the pass has fewer than two workgroups per CU.
 struct Limits {
   size_t lds;
   int threads;
@@ -35,18 +38,22 @@ struct Limits {
 // [N][inner]; ycount = gridDim.y (components)
 // ntables: lookup tables of length N the kernel stages in LDS (N <= 1024);
 // table_elems >= 0 gives the LDS table elements exactly instead
-// min_threads: strided passes of fewer columns than that many threads hold
-// take workgroups of that size all the same (their spare columns are invalid)
+// min_threads: a strided pass that holds all its columns in one workgroup
+// takes a multiple of that many threads (the spare columns are invalid):
+// kernels that sum over a workgroup need whole wavefronts
 PassCfg make_pass_cfg(int N, int rm, long long inner, long long outer, int ycount, size_t max_lds,
                       int ntables = 1, int max_threads = 256, long long table_elems = -1, int min_threads = 0);
 // the same within Limits (max_threads: the kernel's launch bounds)
 inline PassCfg make_pass_cfg(int N, int rm, long long inner, long long outer, int ycount, const Limits& lim,
                              int ntables = 1, int max_threads = 256, long long table_elems = -1, int min_threads = 0) {
+  const int P = threads_per_pencil(N, rm);
   int t = max_threads;
   if (lim.threads > 0) {
-    const int P = threads_per_pencil(N, rm);
     t = lim.threads < max_threads ? lim.threads : max_threads;
     if (t < P) t = P < max_threads ? P : max_threads;
+  } else {
+    const long long pencils = inner * outer * ycount;
+    while (t > 64 && t > P && pencils * P < 2LL * CU_COUNT * t) t >>= 1;
   }
   return make_pass_cfg(N, rm, inner, outer, ycount, lim.lds, ntables, t, table_elems, min_threads);
 }

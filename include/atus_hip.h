@@ -250,13 +250,13 @@ int atus_run_block_profiled(atus_ctx *ctx, const atus_step_params *sp, int Nk, d
 
 /* tuning: values per thread (8 or 16) of the FFT kernels of one kernel
  * family (ATUS_KFAM_*; the Sobolev minimiser's iteration takes 8 always).  16 halves
- * the LDS exchanges, 8 halves the registers per thread.  Defaults: 16 for
- * the contiguous passes and the kinetic step, 8 for the strided passes and
- * the fused V pass. */
+ * the LDS exchanges, 8 halves the registers per thread.  Defaults: 8 for
+ * the strided passes and the fused V pass, and for the contiguous passes
+ * and the kinetic step 16, or 8 below 2^21 values of state. */
 int atus_tune(atus_ctx *ctx, int family, int values_per_thread);
 /* tile choice of a kernel family (no reference counterpart): at most
- * `threads` threads per workgroup (64, 128, 256 or 512; 0 = as many as the
- * kernel allows, the default), i.e. threads / (N / values_per_thread)
+ * `threads` threads per workgroup (64, 128, 256 or 512; 0, the default: as
+ * many as the kernel allows, fewer while that leaves CUs idle), i.e. threads / (N / values_per_thread)
  * pencils per workgroup, at least one.  Fewer pencils per workgroup need
  * less LDS, so more workgroups fit a CU, but strided passes then read rows
  * in shorter segments.  The results do not change. */
