@@ -1180,9 +1180,10 @@ int block_tables(atus_ctx* c, size_t n) {
   return ATUS_OK;
 }
 
-// whether a block of this context runs as one k_block1d launch
-bool resident_ok(const atus_ctx* c) {
-  return c->resident && c->dim == 1 && !c->fs && c->n[0] <= 4096;
+// whether a block of this context (V step vk) runs as one launch
+bool resident_ok(const atus_ctx* c, int vk) {
+  if (!c->resident || c->dim != 1 || c->fs || c->n[0] > 4096) return false;
+  return bcomp_ok(c->n[0], vk, c->nc_run) || (!c->alpha2_set && block1d_ok(c->n[0], vk, c->nc_run));
 }
 
 // a 1D block in one launch: the t1 (and, for a single run, the amplitude)
@@ -1192,11 +1193,11 @@ bool resident_ok(const atus_ctx* c) {
 // fd.fdev
 int resident_block(atus_ctx* c, int vk, const VArgs& base, int Nk, double dt, double* t, const StepFeed& fd,
                    bool batch) {
-  const int N0 = c->n[0];
+  const int N0 = c->n[0], nc = c->nc_run;
+  const long long runs = batch ? c->nbatch : 1;
   double tt = *t + 0.5 * dt;
-  const double* t1tab = fd.t1dev;
-  const double* Ftab = batch ? fd.fbatch : fd.fdev;
-  if (!t1tab) {
+  BlockSteps st{fd.t1dev, batch ? fd.fbatch : fd.fdev, Nk};
+  if (!st.t1) {
     ATUS_TRY(block_tables(c, 2 * (size_t)Nk));
     double tc = tt;
     for (int m = 1; m <= Nk; ++m) {
@@ -1213,32 +1214,88 @@ int resident_block(atus_ctx* c, int vk, const VArgs& base, int Nk, double dt, do
     HIP_TRY(hipMemcpyAsync(c->blk_dev, c->blk_host, sizeof(double) * (batch ? Nk : 2 * Nk), hipMemcpyHostToDevice,
                            c->stream));
     HIP_TRY(hipEventRecord(c->blk_ev, c->stream));
-    t1tab = c->blk_dev;
-    if (!batch) Ftab = c->blk_dev + Nk;
+    st.t1 = c->blk_dev;
+    if (!batch) st.F = c->blk_dev + Nk;
   }
-  if (!t1tab || !Ftab || (batch && !base.runs)) return fail(ATUS_ERR_STATE, "resident block without its step tables");
-  // 8 values per thread: a run's pencil gets the most threads to hide
-  // latency with (4096 points, one run: 10.7 us per step against 13.3 at
-  // 16), and a batch's runs take the plan of the same run alone
-  const int rm = 8;
+  if (!st.t1 || !st.F || (batch && !base.runs)) return fail(ATUS_ERR_STATE, "resident block without its step tables");
+  const KinTabs half = kin_tabs(c, 0), full = kin_tabs(c, 1);
   {
     ProfScope ps(c, ATUS_KFAM_KIN, Nk + 1.0);
-    HIP_TRY(launch_block1d(N0, rm, vk, batch ? 2 : c->ncomp, batch, c->psi, c->npts,
-                           batch ? c->nbatch : 1, c->tw[N0], kin_tabs(c, 0).e0, kin_tabs(c, 1).e0, base, t1tab, Ftab,
-                           c->dx[0], Nk, lim(c, ATUS_KFAM_KIN), c->stream));
+    if (bcomp_ok(N0, vk, nc)) {
+      const BlockPhases ph{{half.e0, half.f0}, {full.e0, full.f0}, half.f0 ? half.split : nc};
+      HIP_TRY(launch_bcomp(N0, vk, nc, batch, c->psi, c->npts, runs, c->tw[N0], ph, base, st, c->dx[0],
+                           lim(c, ATUS_KFAM_KIN), c->stream));
+    } else {
+      HIP_TRY(launch_block1d(vk, batch, c->psi, c->npts, runs, c->tw[N0], half.e0, full.e0, base, st.t1, st.F, c->dx[0],
+                             Nk, lim(c, ATUS_KFAM_KIN), c->stream));
+    }
   }
   for (int m = 1; m <= Nk; ++m) tt += (m < Nk) ? dt : 0.5 * dt;
   *t = tt;
   return ATUS_OK;
 }
 
+// whether a block's V step runs inside the pass along the last axis with
+// the components side by side (k_vcomp): the steps k_vfuse does not cover
+bool vcomp_block_ok(const atus_ctx* c, int vk) {
+  // the numerical exponentials are long chains per point: below 2^17 points
+  // a pass of one thread per point fills the CUs better with them (256^2,
+  // three states: 33 us per step as separate passes, 37 fused; 64x32x64,
+  // four states: 61 and 48)
+  const bool numerical = vk == V_NUM_BRAGG || vk == V_RAMAN;
+  return c->dim >= 2 && (!numerical || c->npts >= (1 << 17)) && vcomp_ok(c->n[c->dim - 1], vk, c->ncomp);
+}
+
+// a block of 2D/3D runs whose V step k_vcomp fuses into the last axis's
+// pass: between two kinetic steps along axis 0 a step is [middle axis
+// inverse (3D), k_vcomp, middle axis forward], the kinetic step's own
+// transforms along those axes; the operations and their order are those of
+// separate V and kinetic steps
+int vcomp_block(atus_ctx* c, int vk, const VArgs& base, int Nk, double dt, double* t, const StepFeed& fd) {
+  const int last = c->dim - 1, NL = c->n[last], N0 = c->n[0];
+  VGeo geo{};
+  geo.dim = c->dim;
+  for (int a = 0; a < 3; ++a) {
+    geo.n[a] = c->n[a];
+    geo.dx[a] = c->dx[a];
+  }
+  VArgs none{};
+  auto kin = [&](int f) -> int {
+    ProfScope ps(c, ATUS_KFAM_KIN);
+    HIP_TRY(launch_kin(N0, vals(c, ATUS_KFAM_KIN), false, V_NONE, 1, c->psi, c->npts, c->ncomp, c->inner_of(0),
+                       c->tw[N0], kin_tabs(c, f), none, c->dx[0], lim(c, ATUS_KFAM_KIN), c->stream));
+    return ATUS_OK;
+  };
+  double tt = *t;
+  for (int a = last; a >= 1; --a) ATUS_TRY(pass(c, a, -1, c->psi, c->psi, c->ncomp, 1.0));
+  ATUS_TRY(kin(0));
+  tt += 0.5 * dt;
+  for (int m = 1; m <= Nk; ++m) {
+    VArgs va;
+    ATUS_TRY(step_vargs(base, m, tt, dt, fd, va));
+    for (int a = 1; a < last; ++a) ATUS_TRY(pass(c, a, +1, c->psi, c->psi, c->ncomp, 1.0));
+    {
+      ProfScope ps(c, ATUS_KFAM_VFUSE);
+      HIP_TRY(launch_vcomp(NL, vk, c->ncomp, c->psi, c->npts, c->npts / NL, c->tw[NL], va, geo,
+                           lim(c, ATUS_KFAM_VFUSE), c->stream));
+    }
+    for (int a = last - 1; a >= 1; --a) ATUS_TRY(pass(c, a, -1, c->psi, c->psi, c->ncomp, 1.0));
+    ATUS_TRY(kin(m < Nk ? 1 : 0));
+    tt += (m < Nk) ? dt : 0.5 * dt;
+  }
+  for (int a = 1; a <= last; ++a) ATUS_TRY(pass(c, a, +1, c->psi, c->psi, c->ncomp, 1.0));
+  *t = tt;
+  return ATUS_OK;
+}
+
 int single_block(atus_ctx* c, int vk, const VArgs& base, int Nk, double dt, double* t, const StepFeed& fd) {
-  // the fused kernels cover one species of up to two components; two
-  // species (per-component kinetic tables, four-component steps) run the
-  // V step and the kinetic step as separate passes
+  // k_vfuse and k_kin cover one species of up to two components; k_vcomp
+  // and k_bcomp the others, up to the lengths their workgroups hold; beyond
+  // those the V step and the kinetic step run as separate passes
   const bool fused = c->ncomp <= 2 && !c->alpha2_set && (vk == V_NL || vk == V_NL_IF || vk == V_BRAGG);
   if (fused && c->dim == 3) return single_block_slabs(c, vk, base, Nk, dt, t, fd);
-  if (fused && !fd.ds && resident_ok(c)) return resident_block(c, vk, base, Nk, dt, t, fd, false);
+  if (resident_ok(c, vk)) return resident_block(c, vk, base, Nk, dt, t, fd, false);
+  if (!fused && vcomp_block_ok(c, vk)) return vcomp_block(c, vk, base, Nk, dt, t, fd);
   const int N0 = c->n[0], NL = c->n[c->dim - 1];
   const long long inner0 = c->inner_of(0);
   double tt = *t;
@@ -1304,7 +1361,7 @@ void batch_vargs(atus_ctx* c, VArgs& base, double dt) {
 // the launches of one block of every run of a batch, without synchronisation
 int batch_block(atus_ctx* c, int vk, const VArgs& base, int Nk, double dt, double* t, const StepFeed& fd) {
   const int B = c->nbatch;
-  if (resident_ok(c)) return resident_block(c, vk, base, Nk, dt, t, fd, true);
+  if (resident_ok(c, vk)) return resident_block(c, vk, base, Nk, dt, t, fd, true);
   const int N0 = c->n[0], NL = c->n[c->dim - 1];
   const long long inner0 = c->inner_of(0);
   double tt = *t;

@@ -1,4 +1,5 @@
-// k_block.hip -- whole blocks of 1D runs in one launch (k_block1d).
+// k_block.hip -- whole blocks of 1D runs of two components and 4096 points in
+// one launch (k_block1d).
 #include "launch.hpp"
 
 namespace atus {
@@ -25,59 +26,27 @@ static hipError_t block_go(double2* psi, long long cs, long long runs, const dou
   return hipGetLastError();
 }
 
-template <int N, int RM>
-static hipError_t block_nr(int vk, int nc, bool batch, double2* psi, long long cs, long long runs,
-                           const double2* tw, const double2* eh, const double2* ef, const VArgs& va,
-                           const double* t1tab, const double* Ftab, double dx0, int Nk, const Limits& max_lds,
-                           hipStream_t s) {
-  if (batch) {
-    if (nc != 2) return hipErrorInvalidValue;
-    if (vk == V_BRAGG)
-      return block_go<N, RM, V_BRAGG, 2, true>(psi, cs, runs, tw, eh, ef, va, t1tab, Ftab, dx0, Nk, max_lds, s);
-    if (vk == V_NL_IF)
-      return block_go<N, RM, V_NL_IF, 2, true>(psi, cs, runs, tw, eh, ef, va, t1tab, Ftab, dx0, Nk, max_lds, s);
-    return hipErrorInvalidValue;
-  }
-  if (nc == 1) {
-    if (vk == V_NL) return block_go<N, RM, V_NL, 1, false>(psi, cs, 1, tw, eh, ef, va, t1tab, Ftab, dx0, Nk, max_lds, s);
-    if (vk == V_NL_IF)
-      return block_go<N, RM, V_NL_IF, 1, false>(psi, cs, 1, tw, eh, ef, va, t1tab, Ftab, dx0, Nk, max_lds, s);
-  } else if (nc == 2) {
-    if (vk == V_NL) return block_go<N, RM, V_NL, 2, false>(psi, cs, 1, tw, eh, ef, va, t1tab, Ftab, dx0, Nk, max_lds, s);
-    if (vk == V_NL_IF)
-      return block_go<N, RM, V_NL_IF, 2, false>(psi, cs, 1, tw, eh, ef, va, t1tab, Ftab, dx0, Nk, max_lds, s);
-    if (vk == V_BRAGG)
-      return block_go<N, RM, V_BRAGG, 2, false>(psi, cs, 1, tw, eh, ef, va, t1tab, Ftab, dx0, Nk, max_lds, s);
-  }
+// two components of 4096 points: a workgroup with a thread group per
+// component would need 1024 threads and spill (a batch of 77 runs: 24 us per
+// step against 11); everything else runs as launch_bcomp
+bool block1d_ok(int N, int vk, int nc) {
+  return N == 4096 && nc == 2 && (vk == V_NL || vk == V_NL_IF || vk == V_BRAGG);
+}
+
+hipError_t launch_block1d(int vk, bool batch, double2* psi, long long cs, long long runs, const double2* tw,
+                          const double2* eh, const double2* ef, const VArgs& va, const double* t1tab,
+                          const double* Ftab, double dx0, int Nk, const Limits& lim, hipStream_t s) {
+  // 8 values per thread: the pencil gets the most threads to hide latency with
+  constexpr int N = 4096, RM = 8;
+  if (vk == V_BRAGG)
+    return batch ? block_go<N, RM, V_BRAGG, 2, true>(psi, cs, runs, tw, eh, ef, va, t1tab, Ftab, dx0, Nk, lim, s)
+                 : block_go<N, RM, V_BRAGG, 2, false>(psi, cs, 1, tw, eh, ef, va, t1tab, Ftab, dx0, Nk, lim, s);
+  if (vk == V_NL_IF)
+    return batch ? block_go<N, RM, V_NL_IF, 2, true>(psi, cs, runs, tw, eh, ef, va, t1tab, Ftab, dx0, Nk, lim, s)
+                 : block_go<N, RM, V_NL_IF, 2, false>(psi, cs, 1, tw, eh, ef, va, t1tab, Ftab, dx0, Nk, lim, s);
+  if (vk == V_NL && !batch)
+    return block_go<N, RM, V_NL, 2, false>(psi, cs, 1, tw, eh, ef, va, t1tab, Ftab, dx0, Nk, lim, s);
   return hipErrorInvalidValue;
-}
-
-// values per thread as tuned for the kinetic family (8 or 16); 8 also at
-// 4096 points, where the per-step kinetic pass falls back to 16
-template <int N>
-static hipError_t block_n(int rm, int vk, int nc, bool batch, double2* psi, long long cs, long long runs,
-                          const double2* tw, const double2* eh, const double2* ef, const VArgs& va,
-                          const double* t1tab, const double* Ftab, double dx0, int Nk, const Limits& max_lds,
-                          hipStream_t s) {
-  if constexpr (N > 8 && N / 8 <= 512) {
-    if (rm == 8) return block_nr<N, 8>(vk, nc, batch, psi, cs, runs, tw, eh, ef, va, t1tab, Ftab, dx0, Nk, max_lds, s);
-  }
-  return block_nr<N, 16>(vk, nc, batch, psi, cs, runs, tw, eh, ef, va, t1tab, Ftab, dx0, Nk, max_lds, s);
-}
-
-hipError_t launch_block1d(int N, int rm, int vk, int nc, bool batch, double2* psi, long long comp_stride,
-                          long long runs, const double2* tw, const double2* eh, const double2* ef, const VArgs& va,
-                          const double* t1tab, const double* Ftab, double dx0, int Nk, const Limits& max_lds,
-                          hipStream_t s) {
-  switch (N) {
-#define ATUS_CASE(n)                                                                                              \
-  case n:                                                                                                         \
-    return block_n<n>(rm, vk, nc, batch, psi, comp_stride, runs, tw, eh, ef, va, t1tab, Ftab, dx0, Nk, max_lds, s);
-    ATUS_CASE(2) ATUS_CASE(4) ATUS_CASE(8) ATUS_CASE(16) ATUS_CASE(32) ATUS_CASE(64) ATUS_CASE(128)
-    ATUS_CASE(256) ATUS_CASE(512) ATUS_CASE(1024) ATUS_CASE(2048) ATUS_CASE(4096)
-#undef ATUS_CASE
-    default: return hipErrorInvalidValue;
-  }
 }
 
 }  // namespace atus

@@ -130,6 +130,76 @@ __device__ __forceinline__ void sincos_fast(double x, double* s, double* c) {
   }
 }
 
+// The same where larger phases are common (kernels whose V step bounds them:
+// the 1D resident blocks, whose potential reaches far from the origin, and
+// the coupled steps of multi.hpp): for |x| < 10^6 a Cody-Waite reduction by n
+// pi/2 (pi/2 = h1 + h2 + h3, the first two of 33 bits, so n h1 and n h2 are
+// exact), then Taylor series to x^19 and x^18 on |r| <= pi/4 (truncation
+// 2e-19 and 2e-18); at most 0.83 ulp off over 2e7 random arguments.  In the
+// passes that stream (k_vfuse) its code costs more than it saves: 2% of the
+// 2048^2 step, 3% of the 32x64x32 one.
+__device__ __forceinline__ void sincos_mid(double x, double* s, double* c) {
+  if (fabs(x) < 0.03125) {
+    const double x2 = x * x;
+    *s = x * (1.0 + x2 * (-1.0 / 6.0 + x2 * (1.0 / 120.0 + x2 * (-1.0 / 5040.0 + x2 * (1.0 / 362880.0 +
+                                                                                  x2 * (-1.0 / 39916800.0))))));
+    *c = 1.0 + x2 * (-0.5 + x2 * (1.0 / 24.0 + x2 * (-1.0 / 720.0 + x2 * (1.0 / 40320.0 + x2 * (-1.0 / 3628800.0)))));
+  } else if (fabs(x) < 1e6) {
+    const double n = rint(x * 0.6366197723675814);
+    // r + rl = x - n pi/2: what each subtraction rounds off is kept in rl
+    const double t = fma(-n, 1.5707963267341256, x), h2 = n * 6.077100506303966e-11;
+    const double u = t - h2;
+    const double r = fma(-n, 2.0222662487959506e-21, u);
+    const double rl = ((t - u) - h2) + fma(-n, 2.0222662487959506e-21, u - r);
+    const double x2 = r * r;
+    double p = -1.0 / 121645100408832000.0;
+    p = fma(p, x2, 1.0 / 355687428096000.0);
+    p = fma(p, x2, -1.0 / 1307674368000.0);
+    p = fma(p, x2, 1.0 / 6227020800.0);
+    p = fma(p, x2, -1.0 / 39916800.0);
+    p = fma(p, x2, 1.0 / 362880.0);
+    p = fma(p, x2, -1.0 / 5040.0);
+    p = fma(p, x2, 1.0 / 120.0);
+    p = fma(p, x2, -1.0 / 6.0);
+    double q = -1.0 / 6402373705728000.0;
+    q = fma(q, x2, 1.0 / 20922789888000.0);
+    q = fma(q, x2, -1.0 / 87178291200.0);
+    q = fma(q, x2, 1.0 / 479001600.0);
+    q = fma(q, x2, -1.0 / 3628800.0);
+    q = fma(q, x2, 1.0 / 40320.0);
+    q = fma(q, x2, -1.0 / 720.0);
+    q = fma(q, x2, 1.0 / 24.0);
+    // sin(r + rl) = r + (r^3 p + rl cos r), cos(r + rl) = (1 - r^2/2) +
+    // (r^4 q - r rl) with the rounding of 1 - r^2/2 added back
+    const double hz = 0.5 * x2, w = 1.0 - hz;
+    const double sr = r + fma(r * x2, p, rl * w);
+    const double cr = w + (((1.0 - w) - hz) + fma(x2 * x2, q, -r * rl));
+    const int k = (int)n;
+    const double a = (k & 1) ? cr : sr, b = (k & 1) ? sr : cr;
+    *s = (k & 2) ? -a : a;
+    *c = ((k + 1) & 2) ? -b : b;
+  } else {
+    sincos(x, s, c);
+  }
+}
+
+template <bool MID>
+__device__ __forceinline__ void sincos_of(double x, double* s, double* c) {
+  if constexpr (MID) sincos_mid(x, s, c);
+  else sincos_fast(x, s, c);
+}
+
+template <bool MID>
+__device__ __forceinline__ double cos_of(double x) {
+  if constexpr (MID) {
+    double s, c;
+    sincos_mid(x, &s, &c);
+    return c;
+  } else {
+    return cos(x);
+  }
+}
+
 // lookup tables (twiddles, kinetic phases) of length N are staged in LDS
 // behind the pencil regions when they are small enough
 template <int N>
@@ -265,7 +335,7 @@ __device__ __forceinline__ void store_pencil(const double2 (&v)[(Plan<N, RM>::R)
 // (CRT_Base_IF.h:381-419) on one point of NC components.  `extra[i]` is the
 // potential V_i (NL, added first as in CRT_Base.h:416) or beta0*x0 - DeltaL_i
 // (NL_IF, added last as in CRT_Base_IF.h:405).
-template <int NC, bool EXTRA_FIRST>
+template <int NC, bool EXTRA_FIRST, bool MID = false>
 __device__ __forceinline__ void nl_point(double2 (&a)[NC], const double (&extra)[NC], const VArgs& p) {
   double phi[NC];
   double n[NC];
@@ -282,7 +352,7 @@ __device__ __forceinline__ void nl_point(double2 (&a)[NC], const double (&extra)
 #pragma unroll
   for (int i = 0; i < NC; ++i) {
     double s, c;
-    sincos_fast(phi[i], &s, &c);
+    sincos_of<MID>(phi[i], &s, &c);
     const double re = a[i].x;
     a[i].x = re * c - a[i].y * s;
     a[i].y = a[i].y * c + re * s;
@@ -290,24 +360,26 @@ __device__ __forceinline__ void nl_point(double2 (&a)[NC], const double (&extra)
 }
 
 // Rabi frequency Omega(x0) and eta(x0) of Do_Bragg_ad (bragg.cpp:224,240)
+template <bool MID = false>
 __device__ __forceinline__ void bragg_field(double x0, const VArgs& p, double& Om, double2& eta) {
   const double t1 = p.t1p ? *p.t1p : p.t1;
   const double F = p.Fp ? *p.Fp : p.F;
   Om = F * p.amp0 *
-       cos(p.laser_k * x0 - (p.laser_domh + p.chirp * t1 + p.chirp_rate0 * t1) * t1 + p.phase0 / 2);
+       cos_of<MID>(p.laser_k * x0 - (p.laser_domh + p.chirp * t1 + p.chirp_rate0 * t1) * t1 + p.phase0 / 2);
   const double arg = -0.5 * (p.laser_dk * x0);
   if (p.laser_dk == 0.0) {
     // arg is +-0: cos = 1 and sin = arg exactly (the sign of zero kept)
     eta = make_double2(1.0, arg);
   } else {
     double s, c;
-    sincos(arg, &s, &c);
+    sincos_of<MID>(arg, &s, &c);
     eta = make_double2(c, s);
   }
 }
 
 // per-point analytic 2x2 exponential of Do_Bragg_ad (bragg.cpp:226-301),
 // same operation order as the reference
+template <bool MID = false>
 __device__ __forceinline__ void bragg_point(double2& a, double2& b, double bx, double Om, double2 eta,
                                             const VArgs& p) {
   const double dt = p.dt;
@@ -317,11 +389,11 @@ __device__ __forceinline__ void bragg_point(double2& a, double2& b, double bx, d
   const double V22 = p.gs[2] * n1 + p.gs[3] * n2 - p.deltaL[1] + bx;
   double s, c;
   if (Om == 0.0) {
-    sincos_fast(-dt * V11, &s, &c);
+    sincos_of<MID>(-dt * V11, &s, &c);
     double re = a.x;
     a.x = re * c - a.y * s;
     a.y = re * s + a.y * c;
-    sincos_fast(-dt * V22, &s, &c);
+    sincos_of<MID>(-dt * V22, &s, &c);
     re = b.x;
     b.x = re * c - b.y * s;
     b.y = re * s + b.y * c;
@@ -330,10 +402,10 @@ __device__ __forceinline__ void bragg_point(double2& a, double2& b, double bx, d
   const double r = sqrt((V11 - V22) * (V11 - V22) + 4.0 * Om * Om);
   const double Ep = 0.5 * (V11 + V22 + r);
   const double Em = 0.5 * (V11 + V22 - r);
-  sincos_fast(-dt * Ep, &s, &c);
+  sincos_of<MID>(-dt * Ep, &s, &c);
   double nrm = 1.0 / fabs((V11 - Ep) * (V11 - Ep) + Om * Om);
   const double gpr = nrm * c, gpi = nrm * s;
-  sincos_fast(-dt * Em, &s, &c);
+  sincos_of<MID>(-dt * Em, &s, &c);
   nrm = 1.0 / fabs((V11 - Em) * (V11 - Em) + Om * Om);
   const double gmr = nrm * c, gmi = nrm * s;
   const double o2 = Om * Om;
@@ -358,15 +430,15 @@ __device__ __forceinline__ void bragg_point(double2& a, double2& b, double bx, d
 __device__ __forceinline__ void ds_pair(double2& a, double2& b, double V11, double V22, double Om, double theta,
                                         double dt) {
   double ei, er;
-  sincos(theta, &ei, &er);
+  sincos_mid(theta, &ei, &er);
   const double tmp1 = sqrt((V11 - V22) * (V11 - V22) + 4.0 * Om * Om);
   const double Ep = 0.5 * (V11 + V22 + tmp1);
   const double Em = 0.5 * (V11 + V22 - tmp1);
   const double d0 = V11 - Ep, d1 = V11 - Em;
   const double den0 = fabs(d0 * d0 + Om * Om), den1 = fabs(d1 * d1 + Om * Om);
   double s0, c0, s1, c1;
-  sincos(-dt * Ep, &s0, &c0);
-  sincos(-dt * Em, &s1, &c1);
+  sincos_mid(-dt * Ep, &s0, &c0);
+  sincos_mid(-dt * Em, &s1, &c1);
   const double g0r = c0 / den0, g0i = s0 / den0, g1r = c1 / den1, g1i = s1 / den1;
   const double tr = d0 * g0r + d1 * g1r, ti = d0 * g0i + d1 * g1i;
   const double o2 = Om * Om;
@@ -386,7 +458,7 @@ __device__ __forceinline__ void ds_pair(double2& a, double2& b, double V11, doub
 
 __device__ __forceinline__ void ds_diag(double2& a, double phi, double dt) {
   double im1, re1;
-  sincos(-phi * dt, &im1, &re1);
+  sincos_mid(-phi * dt, &im1, &re1);
   const double tmp1 = a.x;
   a.x = tmp1 * re1 - a.y * im1;
   a.y = tmp1 * im1 + a.y * re1;
@@ -408,8 +480,8 @@ __device__ __forceinline__ void bragg_ds_point(double2 (&a)[4], double x0, const
     phi[i] = ph;
   }
   const double t1 = p.t1p ? *p.t1p : p.t1;
-  const double Om = p.mode1 * p.amp0 * cos(p.laser_k * x0 - (p.laser_domh + p.chirp_rate0 * t1) * t1 + p.phase0 / 2);
-  const double Om2 = p.mode2 * p.amp2 * cos(p.laser_k2 * x0 - (p.laser_domh2 + p.chirp_rate2 * t1) * t1 + p.phase2 / 2);
+  const double Om = p.mode1 * p.amp0 * cos_of<true>(p.laser_k * x0 - (p.laser_domh + p.chirp_rate0 * t1) * t1 + p.phase0 / 2);
+  const double Om2 = p.mode2 * p.amp2 * cos_of<true>(p.laser_k2 * x0 - (p.laser_domh2 + p.chirp_rate2 * t1) * t1 + p.phase2 / 2);
   const double th1 = -0.5 * (p.laser_dk * x0 + p.phase0);
   const double th2 = -0.5 * (p.laser_dk2 * x0 + p.phase2);
   if (Om == 0.0 && Om2 == 0.0) {
@@ -431,28 +503,28 @@ __device__ __forceinline__ void bragg_ds_point(double2 (&a)[4], double x0, const
 
 // V step on the registers of NC component pencils at one element.
 // x0: first-axis coordinate of the element; l: linear point index.
-template <int VK, int NC>
+template <int VK, int NC, bool MID = false>
 __device__ __forceinline__ void v_point(double2 (&a)[NC], double x0, long long l, const VArgs& p,
                                         double Om, double2 eta) {
   if constexpr (VK == V_NL) {
     double extra[NC];
 #pragma unroll
     for (int c = 0; c < NC; ++c) extra[c] = p.pot ? p.pot[c * p.pot_stride + l] : 0.0;
-    nl_point<NC, true>(a, extra, p);
+    nl_point<NC, true, MID>(a, extra, p);
   } else if constexpr (VK == V_NL_IF) {
     double extra[NC];
 #pragma unroll
     for (int c = 0; c < NC; ++c) extra[c] = p.beta0 * x0 - p.deltaL[c];
-    nl_point<NC, false>(a, extra, p);
+    nl_point<NC, false, MID>(a, extra, p);
   } else if constexpr (VK == V_BRAGG) {
     static_assert(NC == 2, "Bragg coupling needs two components");
-    bragg_point(a[0], a[1], p.beta0 * x0, Om, eta, p);
+    bragg_point<MID>(a[0], a[1], p.beta0 * x0, Om, eta, p);
   } else if constexpr (VK == V_NL_IF2) {
     // CRT_Base_IF_2::Do_NL_Step (CRT_Base_IF_2.h:324-366)
     double extra[NC];
 #pragma unroll
     for (int c = 0; c < NC; ++c) extra[c] = (c < NC / 2 ? p.beta0 : p.beta2) * x0 - p.deltaL[c];
-    nl_point<NC, false>(a, extra, p);
+    nl_point<NC, false, MID>(a, extra, p);
   } else if constexpr (VK == V_BRAGG_DS) {
     static_assert(NC == 4, "the two-species Bragg step has four components");
     bragg_ds_point(a, x0, p);
@@ -536,7 +608,7 @@ __device__ __forceinline__ void herm_expm_apply(double2 (&H)[N][N], double dt, d
       acc.y += V[k][i].x * psi[k].y - V[k][i].y * psi[k].x;
     }
     double sn, cs;
-    sincos(-dt * H[i][i].x, &sn, &cs);
+    sincos_mid(-dt * H[i][i].x, &sn, &cs);
     y[i] = cmul(acc, make_double2(cs, sn));
   }
 #pragma unroll
@@ -582,7 +654,7 @@ __device__ __forceinline__ void num_bragg_point(double2 (&a)[NC], double x0, dou
     const double k = i == 0 ? p.laser_k : -p.laser_k;
     const double cr = i == 0 ? p.chirp_rate0 : -p.chirp_rate0;
     double sn, cs;
-    sincos((-p.laser_domh + cr * t) * t + k * x0 - 0.5 * p.phase0, &sn, &cs);
+    sincos_mid((-p.laser_domh + cr * t) * t + k * x0 - 0.5 * p.phase0, &sn, &cs);
     const double er = p.amp0 * cs / 2 + p.amp1 * cs / 2;
     const double ei = p.amp0 * sn / 2 - p.amp1 * sn / 2;
     H[i + 1][0] = make_double2(er, ei);
@@ -600,7 +672,7 @@ __device__ __forceinline__ void raman_point(double2 (&a)[NC], double x0, double 
   three_state_diag<NC>(H, a, bx, p);
   H[2][2].x = H[2][2].x + p.laser_domh;
   double sn, cs;
-  sincos(p.laser_k * x0, &sn, &cs);
+  sincos_mid(p.laser_k * x0, &sn, &cs);
   H[0][2] = make_double2(p.amp0 / 2 * cs, p.amp0 / 2 * sn);
   H[2][0] = make_double2(p.amp0 / 2 * cs, -(p.amp0 / 2 * sn));
   H[1][2] = make_double2(p.amp1 / 2 * cs, -(p.amp1 / 2 * sn));
@@ -620,16 +692,16 @@ __device__ __forceinline__ void dbragg_point(double2 (&a)[3], double x0, double 
   const double V11 = p.gs[0] * n1 + p.gs[1] * n2 + p.gs[2] * n3 + bx;
   const double V22 = p.gs[3] * n1 + p.gs[4] * n2 + p.gs[5] * n3 - p.deltaL[1] + bx;
   double dw = p.laser_domh + p.chirp_rate0 * t1;
-  const double Op = F * p.amp0 * cos(p.laser_k * x0 - dw * t1 - p.phase0 / 2);
+  const double Op = F * p.amp0 * cos_of<true>(p.laser_k * x0 - dw * t1 - p.phase0 / 2);
   dw = p.laser_domh - p.chirp_rate0 * t1;
-  const double Om = F * p.amp0 * cos(-p.laser_k * x0 - dw * t1 - p.phase0 / 2);
+  const double Om = F * p.amp0 * cos_of<true>(-p.laser_k * x0 - dw * t1 - p.phase0 / 2);
   double im1, re1, tmp1, tmp2;
   if (Om == 0.0 && Op == 0.0) {
-    sincos(-dt * V11, &im1, &re1);
+    sincos_mid(-dt * V11, &im1, &re1);
     tmp1 = a[0].x;
     a[0].x = tmp1 * re1 - a[0].y * im1;
     a[0].y = tmp1 * im1 + a[0].y * re1;
-    sincos(-dt * V22, &im1, &re1);
+    sincos_mid(-dt * V22, &im1, &re1);
 #pragma unroll
     for (int c = 1; c < 3; ++c) {
       tmp1 = a[c].x;
@@ -638,18 +710,18 @@ __device__ __forceinline__ void dbragg_point(double2 (&a)[3], double x0, double 
     }
     return;
   }
-  sincos(-0.5 * p.laser_dk * x0, &im1, &re1);
+  sincos_mid(-0.5 * p.laser_dk * x0, &im1, &re1);
   const double e0 = re1, e1 = im1;
   tmp1 = sqrt((V11 - V22) * (V11 - V22) + 4.0 * (Op * Op + Om * Om));
   const double E1 = 0.5 * (V11 + V22 + tmp1);
   const double E2 = 0.5 * (V11 + V22 - tmp1);
-  sincos(-dt * E1, &im1, &re1);
+  sincos_mid(-dt * E1, &im1, &re1);
   tmp1 = 1.0 / fabs((V22 - E1) * (V22 - E1) + Op * Op + Om * Om);
   const double g1r = tmp1 * re1, g1i = tmp1 * im1;
-  sincos(-dt * E2, &im1, &re1);
+  sincos_mid(-dt * E2, &im1, &re1);
   tmp1 = 1.0 / fabs((V22 - E2) * (V22 - E2) + Op * Op + Om * Om);
   const double g2r = tmp1 * re1, g2i = tmp1 * im1;
-  sincos(-dt * V22, &im1, &re1);
+  sincos_mid(-dt * V22, &im1, &re1);
   tmp1 = 1.0 / fabs(Op * Op + Om * Om);
   const double g3r = tmp1 * re1, g3i = tmp1 * im1;
   tmp1 = (V22 - E2) * (V22 - E2);
@@ -821,7 +893,9 @@ __global__ __launch_bounds__(LB) void k_kin(double2* __restrict__ psi, long long
 
 // ------------------------------------------------------------ k_block1d
 // A whole block of 1D runs in one launch (N <= 4096: each run's pencil
-// stays in the registers of its threads for all Nk steps): the half
+// stays in the registers of its threads for all Nk steps, both components of
+// a point in one thread; k_bcomp covers one component and, up to 2048
+// points, spreads several over thread groups): the half
 // kinetic step, then Nk times the V step followed by the full kinetic step
 // (the last one half), as the eager block launches them, with k_kin's
 // operations (transform, V step, phase multiply).  The results agree with
@@ -864,37 +938,14 @@ __global__ __launch_bounds__(LB) void k_block1d(double2* __restrict__ psi, long 
   for (int c = 0; c < NC; ++c) load_pencil<N, RM>(v[c], psi + c0 + c * comp_stride, m.base, 1, m.t, m.valid);
   __syncthreads();
   auto kinetic = [&](const double2* e) {
-    if constexpr (NC == 1 && !tables_in_lds<N>()) {
-      // phases from global memory: loaded before the forward transform,
-      // whose barriers the loads could not otherwise move across
-      double2 ev[R];
-#pragma unroll
-      for (int i = 0; i < R; ++i) ev[i] = e[m.t + P * i];
-      fft_pencil<N, RM, -1, WAVE>(v[0], m.t, lds, twl);
-#pragma unroll
-      for (int i = 0; i < R; ++i) v[0][i] = cmul(v[0][i], ev[i]);
-      fft_pencil<N, RM, +1, WAVE>(v[0], m.t, lds, twl);
-    } else {
-#pragma unroll
-      for (int c = 0; c < NC; ++c) {
-        fft_pencil<N, RM, -1, WAVE>(v[c], m.t, lds, twl);
-#pragma unroll
-        for (int i = 0; i < R; ++i) v[c][i] = cmul(v[c][i], e[m.t + P * i]);
-        fft_pencil<N, RM, +1, WAVE>(v[c], m.t, lds, twl);
-      }
-    }
-  };
-  // the potential is the same for every step of the block: read once into
-  // registers rather than after every step's last barrier
-  double potv[VK == V_NL ? NC : 1][VK == V_NL ? R : 1];
-  if constexpr (VK == V_NL) {
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
+      fft_pencil<N, RM, -1, WAVE>(v[c], m.t, lds, twl);
 #pragma unroll
-      for (int i = 0; i < R; ++i)
-        potv[c][i] = (va.pot && m.valid) ? va.pot[c * va.pot_stride + m.base + m.t + P * i] : 0.0;
+      for (int i = 0; i < R; ++i) v[c][i] = cmul(v[c][i], e[m.t + P * i]);
+      fft_pencil<N, RM, +1, WAVE>(v[c], m.t, lds, twl);
     }
-  }
+  };
   kinetic(ehl);
   for (int s = 1; s <= Nk; ++s) {
     va.t1p = t1tab + (s - 1);
@@ -914,15 +965,7 @@ __global__ __launch_bounds__(LB) void k_block1d(double2* __restrict__ psi, long 
       double Om = 0.0;
       double2 eta = make_double2(1.0, 0.0);
       if constexpr (VK == V_BRAGG) bragg_field(x0, va, Om, eta);
-      if constexpr (VK == V_NL) {
-        // v_point's V_NL branch with the preloaded potential
-        double extra[NC];
-#pragma unroll
-        for (int c = 0; c < NC; ++c) extra[c] = potv[c][i];
-        if (m.valid) nl_point<NC, true>(a, extra, va);
-      } else {
-        if (m.valid) v_point<VK, NC>(a, x0, m.base + j, va, Om, eta);
-      }
+      if (m.valid) v_point<VK, NC>(a, x0, m.base + j, va, Om, eta);
 #pragma unroll
       for (int c = 0; c < NC; ++c) v[c][i] = a[c];
     }

@@ -7,6 +7,27 @@
 
 namespace atus {
 
+// geometry of the multi-component pass along the last axis
+struct VGeo {
+  int dim;
+  int n[3];
+  double dx[3];
+};
+// per-step values of a resident block: t1 and the amplitude (single runs
+// [Nk], batches [Nk][runs])
+struct BlockSteps {
+  const double* t1;
+  const double* F;
+  int Nk;
+};
+// half and full kinetic phases of a 1D grid; components from `split` on take
+// the second pair
+struct BlockPhases {
+  const double2* half[2];
+  const double2* full[2];
+  int split;
+};
+
 struct SobTurn;
 struct SobMix;
 struct SobFinish;
@@ -101,14 +122,26 @@ hipError_t launch_vstep_batch(int N, int rm, bool one_d, int vk, double2* psi, l
                               double dx0, const Limits& max_lds, hipStream_t s, const double2* kz = nullptr,
                               int edge = 0);
 
-// a whole block of a 1D grid (N <= 4096) in one launch: one run (nc
-// components, runs = 1) or a batch of `runs` two-component runs; eh / ef
-// the half and full kinetic phase tables, t1tab [Nk] and Ftab ([Nk] or
-// [Nk][runs]) the per-step t1 and amplitudes in device memory
-hipError_t launch_block1d(int N, int rm, int vk, int nc, bool batch, double2* psi, long long comp_stride,
-                          long long runs, const double2* tw, const double2* eh, const double2* ef, const VArgs& va,
-                          const double* t1tab, const double* Ftab, double dx0, int Nk, const Limits& max_lds,
-                          hipStream_t s);
+// a whole block of two components of 4096 points in one launch: one run
+// (runs = 1) or a batch of `runs`; eh / ef the half and full kinetic phase
+// tables, t1tab [Nk] and Ftab ([Nk] or [Nk][runs]) the per-step t1 and
+// amplitudes in device memory
+bool block1d_ok(int N, int vk, int nc);
+hipError_t launch_block1d(int vk, bool batch, double2* psi, long long cs, long long runs, const double2* tw,
+                          const double2* eh, const double2* ef, const VArgs& va, const double* t1tab,
+                          const double* Ftab, double dx0, int Nk, const Limits& lim, hipStream_t s);
+
+// the same passes with the components on thread groups of their own
+// (multi.hpp); *_ok: whether the kind, component count and length are
+// covered.  launch_vcomp: inverse / V / forward along the last axis of a
+// 2D/3D grid, `outer` pencils; launch_bcomp: blocks of 1D runs
+bool vcomp_ok(int N, int vk, int nc);
+hipError_t launch_vcomp(int N, int vk, int nc, double2* psi, long long comp_stride, long long outer,
+                        const double2* tw, const VArgs& va, const VGeo& geo, const Limits& lim, hipStream_t s);
+bool bcomp_ok(int N, int vk, int nc);
+hipError_t launch_bcomp(int N, int vk, int nc, bool batch, double2* psi, long long comp_stride, long long runs,
+                        const double2* tw, const BlockPhases& ph, const VArgs& va, const BlockSteps& st, double dx0,
+                        const Limits& lim, hipStream_t s);
 
 // column pass of the four-step 1D transform (k_fs_col): n1 in 64..1024,
 // mode FS_ENTER / FS_EXIT / FS_STEP; ycount components (NC == 1, no
