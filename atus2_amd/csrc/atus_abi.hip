@@ -519,6 +519,93 @@ int reduce_seg(atus_ctx* c, const Fn& fn, long long n, long long seg_stride, int
   return reduce_seg_into(c, fn, n, seg_stride, nseg, nb, c->sred_part, c->sred_out, out);
 }
 
+// Densities along every axis of one component at p (launch_marginal), for
+// grids without a four-step axis: x[a][j] is the sum of
+// |psi|^2 and k[a][j] that of |psi^|^2 (psi^ with ft's factor) over the
+// other axes.  phase: also the sum of atan2(Im, Re) |psi|^2.  One
+// synchronisation in all.
+struct Marginals {
+  std::vector<double> x[3], k[3];
+  double phase = 0;
+  // sum of f(coordinate) times the density
+  static double moment(const std::vector<double>& d, const std::vector<double>& q, double mu, int power) {
+    double s = 0.0;
+    for (size_t j = 0; j < d.size(); ++j) {
+      const double e = q[j] - mu;
+      s += d[j] * (power == 0 ? 1.0 : power == 1 ? e : e * e);
+    }
+    return s;
+  }
+};
+
+std::vector<double> axis_x(const atus_ctx* c, int a) {
+  std::vector<double> q(c->n[a]);
+  for (int j = 0; j < c->n[a]; ++j) q[j] = (double)(j - c->n[a] / 2) * c->dx[a];
+  return q;
+}
+
+std::vector<double> axis_k(const atus_ctx* c, int a) {
+  std::vector<double> q(c->n[a]);
+  const int n = c->n[a], sh = n / 2;
+  for (int j = 0; j < n; ++j) q[j] = c->dk[a] * (double)(((j + sh) % n) - sh);
+  return q;
+}
+
+int marginals(atus_ctx* c, const double2* p, bool phase, Marginals& m) {
+  size_t npart = 0, nout = 0;
+  unsigned nb[3] = {0, 0, 0};
+  for (int a = 0; a < c->dim; ++a) {
+    ATUS_TRY(ensure_twiddles(c, c->n[a]));
+    const int fam = a == c->dim - 1 ? ATUS_KFAM_PASS_CONTIG : ATUS_KFAM_PASS_STRIDED;
+    HIP_TRY(launch_marginal(c->n[a], nullptr, c->inner_of(a), c->outer_of(a), nullptr, nullptr, nullptr, nullptr, &nb[a],
+                            lim(c, fam), c->stream));
+    npart = std::max(npart, (size_t)nb[a] * c->n[a]);
+    nout += c->n[a];
+  }
+  const size_t nph = phase ? nb[c->dim - 1] : 0;
+  const size_t need = 2 * (npart + nout) + nph + 1;
+  if (c->marg_cap < need) {
+    HIP_TRY(hipStreamSynchronize(c->stream));
+    (void)hipFree(c->marg);
+    c->marg = nullptr;
+    c->marg_cap = 0;
+    if (hipMalloc(&c->marg, sizeof(double) * need) != hipSuccess) return fail(ATUS_ERR_NOMEM, "density buffers");
+    c->marg_cap = need;
+  }
+  // [axis 0][axis 1][axis 2][phase partials], then the partial sums of one
+  // axis at a time (a stream's passes follow each other)
+  double* out = c->marg;
+  double* ph = out + 2 * nout;
+  double2* part = (double2*)(ph + nph + ((nph & 1) ? 1 : 0));
+  size_t o = 0;
+  for (int a = 0; a < c->dim; ++a) {
+    const bool last = a == c->dim - 1;
+    HIP_TRY(launch_marginal(c->n[a], p, c->inner_of(a), c->outer_of(a), c->tw[c->n[a]], part, (double2*)(out + 2 * o),
+                            phase && last ? ph : nullptr, &nb[a],
+                            lim(c, last ? ATUS_KFAM_PASS_CONTIG : ATUS_KFAM_PASS_STRIDED), c->stream));
+    o += c->n[a];
+  }
+  std::vector<double> h(2 * nout + nph);
+  HIP_TRY(hipMemcpyAsync(h.data(), out, sizeof(double) * h.size(), hipMemcpyDeviceToHost, c->stream));
+  HIP_TRY(hipStreamSynchronize(c->stream));
+  const double f = ft_factor(c->dim, c->dx);
+  o = 0;
+  for (int a = 0; a < c->dim; ++a) {
+    const int n = c->n[a];
+    const double w = f * f * ((double)c->npts / n);  // the other axes' transforms
+    m.x[a].resize(n);
+    m.k[a].resize(n);
+    for (int j = 0; j < n; ++j) {
+      m.x[a][j] = h[2 * (o + j)];
+      m.k[a][j] = w * h[2 * (o + j) + 1];
+    }
+    o += n;
+  }
+  m.phase = 0;
+  for (size_t b = 0; b < nph; ++b) m.phase += h[2 * nout + b];
+  return ATUS_OK;
+}
+
 // The Rabi integrals' reduction (RedRabi): over the index box of the balls
 // |k - k0_q| < thr when that box is under half the grid (RedRabiBox, the
 // same sums over far fewer points), else over every point.  Per axis the
@@ -827,7 +914,7 @@ int atus_ctx_destroy(atus_ctx* c) {
   (void)hipFree(c->red_out);
   if (c->red_host) (void)hipHostFree(c->red_host);
   (void)hipFree(c->sob);
-  (void)hipFree(c->lap);
+  (void)hipFree(c->marg);
   (void)hipFree(c->sob_st);
   (void)hipFree(c->sob_part);
   (void)hipFree(c->sob_log);
@@ -1569,8 +1656,16 @@ int atus_expval_x(atus_ctx* c, int comp, double out[3]) {
 int atus_expval_k(atus_ctx* c, int comp, double out[3]) {
   ATUS_TRY(check_ctx(c));
   ATUS_TRY(check_comp(c, comp));
+  const double2* p = c->psi + comp * c->npts;
+  if (!c->fs) {
+    Marginals m;
+    ATUS_TRY(marginals(c, p, false, m));
+    for (int a = 0; a < 3; ++a)
+      out[a] = a < c->dim ? c->ar_k() * Marginals::moment(m.k[a], axis_k(c, a), 0.0, 1) : 0.0;
+    return ATUS_OK;
+  }
   ATUS_TRY(ensure_scratch(c));
-  ATUS_TRY(full_ft(c, -1, c->psi + comp * c->npts, c->scratch, 1));
+  ATUS_TRY(full_ft(c, -1, p, c->scratch, 1));
   RedK fn{c->scratch, c->grid()};
   double s[3];
   ATUS_TRY(reduce(c, fn, c->npts, s));
@@ -1585,6 +1680,25 @@ int atus_get_moments(atus_ctx* c, int comp, atus_moments* out) {
   *out = atus_moments{};
   const double2* p = c->psi + comp * c->npts;
   const int D = c->dim;
+  if (!c->fs) {
+    // every moment from the densities along the axes
+    Marginals m;
+    ATUS_TRY(marginals(c, p, true, m));
+    const std::vector<double> x0 = axis_x(c, 0);
+    const double sum = Marginals::moment(m.x[0], x0, 0.0, 0);
+    if (!(sum > 0.0)) return fail(ATUS_ERR_NUMERIC, "the state is zero");
+    const double PN = c->ar() * sum;
+    out->N = PN;
+    out->phase = m.phase / sum;
+    for (int a = 0; a < D; ++a) {
+      const std::vector<double> x = axis_x(c, a), k = axis_k(c, a);
+      out->x[a] = Marginals::moment(m.x[a], x, 0.0, 1) * (c->ar() / PN);
+      out->x2[a] = Marginals::moment(m.x[a], x, out->x[a], 2) * (c->ar() / PN);
+      out->k[a] = Marginals::moment(m.k[a], k, 0.0, 1) * (c->ar_k() / PN);
+      out->k2[a] = Marginals::moment(m.k[a], k, out->k[a], 2) * (c->ar_k() / PN);
+    }
+    return ATUS_OK;
+  }
   double s1[5];
   ATUS_TRY(reduce(c, RedMom1{p, c->grid()}, c->npts, s1));
   if (!(s1[0] > 0.0)) return fail(ATUS_ERR_NUMERIC, "the state is zero");
@@ -1674,27 +1788,39 @@ int atus_energy(atus_ctx* c, double* out) {
   ATUS_TRY(check_ctx(c));
   ATUS_TRY(check_single(c, "atus_energy"));
   if (!out) return fail(ATUS_ERR_ARG, "null output");
-  ATUS_TRY(ensure_scratch(c));
   double ekin = 0;
   for (int i = 0; i < c->ncomp; ++i) {
+    const double* ai = (c->alpha2_set && i >= c->ncomp / 2) ? c->alpha2 : c->alpha;
+    if (!c->fs) {
+      Marginals m;
+      ATUS_TRY(marginals(c, c->psi + i * c->npts, false, m));
+      for (int a = 0; a < c->dim; ++a) ekin += ai[a] * Marginals::moment(m.k[a], axis_k(c, a), 0.0, 2);
+      continue;
+    }
+    ATUS_TRY(ensure_scratch(c));
     ATUS_TRY(full_ft(c, -1, c->psi + i * c->npts, c->scratch, 1));
     RedEkin fn{};
     fn.psik = c->scratch;
     fn.gr = c->grid();
-    const double* al = (c->alpha2_set && i >= c->ncomp / 2) ? c->alpha2 : c->alpha;
-    for (int a = 0; a < 3; ++a) fn.alpha[a] = al[a];
+    for (int a = 0; a < 3; ++a) fn.alpha[a] = ai[a];
     double s;
     ATUS_TRY(reduce(c, fn, c->npts, &s));
     ekin += s;
   }
-  RedEpot fp{};
-  fp.psi = c->psi;
-  fp.pot = c->pot;
-  fp.npts = c->npts;
-  fp.nc = c->ncomp;
-  for (int i = 0; i < 16; ++i) fp.gs[i] = c->gs[i];
-  double ep;
-  ATUS_TRY(reduce(c, fp, c->npts, &ep));
+  double ep = 0;
+  auto epot = [&](auto fp) -> int {
+    fp.psi = c->psi;
+    fp.pot = c->pot;
+    fp.npts = c->npts;
+    for (int i = 0; i < 16; ++i) fp.gs[i] = c->gs[i];
+    return reduce(c, fp, c->npts, &ep);
+  };
+  switch (c->ncomp) {
+    case 1: ATUS_TRY(epot(RedEpot<1>{})); break;
+    case 2: ATUS_TRY(epot(RedEpot<2>{})); break;
+    case 3: ATUS_TRY(epot(RedEpot<3>{})); break;
+    default: ATUS_TRY(epot(RedEpot<4>{})); break;
+  }
   *out = c->ar_k() * ekin + c->ar() * ep;
   return ATUS_OK;
 }
@@ -1702,34 +1828,6 @@ int atus_energy(atus_ctx* c, double* out) {
 // ------------------------------------------------------------------ Sobolev
 
 namespace {
-
-// out_sob = F^-1[op F psi], out_lap = F^-1[-alpha k^2 F psi] (optional)
-int sob_filter(atus_ctx* c, int comp, const double2* src, double2* out_sob, double2* out_lap) {
-  const long long off = comp * c->npts;
-  SobArgs sa{};
-  sa.alpha = c->sob_alpha[comp];
-  sa.dim = c->dim;
-  for (int a = 0; a < 3; ++a) {
-    sa.dk[a] = c->dk[a];
-    sa.n[a] = c->n[a];
-  }
-  sa.scale = ft_factor(c->dim, c->dx) * ft_factor(c->dim, c->dk);
-  const double2* s = src + off;
-  double2* w = out_sob + off;
-  for (int a = c->dim - 1; a >= 1; --a) {
-    ATUS_TRY(pass(c, a, -1, s, w, 1, 1.0));
-    s = w;
-  }
-  const int N0 = c->n[0];
-  ATUS_TRY(ensure_twiddles(c, N0));
-  HIP_TRY(launch_sobf(N0, vals(c, ATUS_KFAM_KIN), c->dim == 1, s, w, out_lap ? out_lap + off : nullptr, c->npts, 1, c->inner_of(0),
-                      c->tw[N0], sa, lim(c, ATUS_KFAM_KIN), c->stream));
-  for (int a = 1; a < c->dim; ++a) {
-    ATUS_TRY(pass(c, a, +1, w, w, 1, 1.0));
-    if (out_lap) ATUS_TRY(pass(c, a, +1, out_lap + off, out_lap + off, 1, 1.0));
-  }
-  return ATUS_OK;
-}
 
 // arguments of the Sobolev loop's kernels
 SobMix sob_mix_args(const atus_ctx* c) {
@@ -1816,10 +1914,10 @@ int sob_loop_line(atus_ctx* c, int count, double eps) {
   return ATUS_OK;
 }
 
+// sum (V + sum_j g_j |psi_j|^2) |psi_comp|^2
 struct RedMu {
   static constexpr int NV = 1;
   const double2* psi;
-  const double2* lap;
   const double* pot;
   long long npts;
   int nw, comp;
@@ -1830,8 +1928,8 @@ struct RedMu {
       const double2 a = psi[j * npts + l];
       nl += (j == 0 ? g0 : g1) * (a.x * a.x + a.y * a.y);
     }
-    const double2 p = psi[comp * npts + l], lp = lap[comp * npts + l];
-    acc[0] += -(p.x * lp.x + p.y * lp.y) + (pot[comp * npts + l] + nl) * (p.x * p.x + p.y * p.y);
+    const double2 p = psi[comp * npts + l];
+    acc[0] += (pot[comp * npts + l] + nl) * (p.x * p.x + p.y * p.y);
   }
 };
 
@@ -1848,7 +1946,6 @@ int atus_sob_setup(atus_ctx* c, const double* alpha_iso, double stepsize) {
   c->sob_step = stepsize;
   const size_t bytes = sizeof(double2) * c->npts * c->ncomp;
   if (!c->sob && hipMalloc(&c->sob, 2 * bytes) != hipSuccess) return fail(ATUS_ERR_NOMEM, "Sobolev buffers");
-  if (!c->lap && hipMalloc(&c->lap, bytes) != hipSuccess) return fail(ATUS_ERR_NOMEM, "Sobolev buffers");
   if ((!c->sob_st && hipMalloc(&c->sob_st, sizeof(SobState)) != hipSuccess) ||
       (!c->sob_log && hipMalloc(&c->sob_log, sizeof(double) * SOB_MAX_CHUNK * SOB_LOG_VALS) != hipSuccess))
     return fail(ATUS_ERR_NOMEM, "Sobolev loop state");
@@ -1910,11 +2007,18 @@ int atus_sob_mu(atus_ctx* c, double* mu) {
   if (!c->sob_ready) return fail(ATUS_ERR_STATE, "call atus_sob_setup first");
   if (!mu) return fail(ATUS_ERR_ARG, "null output");
   const int nw = c->ncomp;
-  for (int i = 0; i < nw; ++i) ATUS_TRY(sob_filter(c, i, c->psi, c->sob, c->lap));
+  // -<psi, Lap psi> = s sum alpha k^2 |F psi|^2 (s the transform pair's
+  // scale): the densities carry ft's forward factor twice instead
+  const double fx = ft_factor(c->dim, c->dx), fk = ft_factor(c->dim, c->dk);
   for (int i = 0; i < nw; ++i) {
-    RedMu fn{c->psi, c->lap, c->pot, c->npts, nw, i, c->gs[0 + i * nw], nw > 1 ? c->gs[1 + i * nw] : 0.0};
+    Marginals m;
+    ATUS_TRY(marginals(c, c->psi + i * c->npts, false, m));
+    double kin = 0.0;
+    for (int a = 0; a < c->dim; ++a) kin += c->sob_alpha[i] * Marginals::moment(m.k[a], axis_k(c, a), 0.0, 2);
+    RedMu fn{c->psi, c->pot, c->npts, nw, i, c->gs[0 + i * nw], nw > 1 ? c->gs[1 + i * nw] : 0.0};
     double s;
     ATUS_TRY(reduce(c, fn, c->npts, &s));
+    s += kin * fk / fx;
     mu[i] = c->ar() * s;
   }
   return ATUS_OK;

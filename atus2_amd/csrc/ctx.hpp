@@ -99,12 +99,15 @@ struct atus_ctx {
   double2* rbuf = nullptr;
   size_t rbuf_cap = 0;
 
+  // densities along the axes: their sums and partial sums
+  double* marg = nullptr;
+  size_t marg_cap = 0;
+
   bool sob_ready = false;
   double sob_alpha[2] = {0, 0};
   double sob_step = 0;
-  // the iteration's spectra [2 ncomp][npts] (k_sob_turn), the Laplacian of
-  // the chemical potential
-  double2 *sob = nullptr, *lap = nullptr;
+  // the iteration's spectra [2 ncomp][npts] (k_sob_turn)
+  double2* sob = nullptr;
   // the device-side loop: its state (atus::SobState), the passes' partial
   // sums and the per-iteration log [SOB_MAX_CHUNK][4]
   void* sob_st = nullptr;

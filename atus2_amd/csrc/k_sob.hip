@@ -4,46 +4,6 @@
 
 namespace atus {
 
-template <int N, int RM>
-static hipError_t sob_nr(bool contig, const double2* src, double2* o1, double2* o2, long long cs, int ncomp,
-                         long long inner, const double2* tw, const SobArgs& sa, const Limits& max_lds, hipStream_t s) {
-  PassCfg c = make_pass_cfg(N, RM, contig ? 1 : inner, 1, ncomp, max_lds);
-  if (c.block.x == 0 || c.block.x > 256 || c.grid.x == 0) return hipErrorInvalidConfiguration;
-  static bool ok[2] = {false, false};
-  hipError_t e;
-  if (contig) {
-    e = allow_lds(k_sobf<N, RM, true>, c.lds, ok[0]);
-    if (e == hipSuccess)
-      hipLaunchKernelGGL((k_sobf<N, RM, true>), c.grid, c.block, c.lds, s, src, o1, o2, cs, c.g, tw, sa);
-  } else {
-    e = allow_lds(k_sobf<N, RM, false>, c.lds, ok[1]);
-    if (e == hipSuccess)
-      hipLaunchKernelGGL((k_sobf<N, RM, false>), c.grid, c.block, c.lds, s, src, o1, o2, cs, c.g, tw, sa);
-  }
-  if (e != hipSuccess) return e;
-  return hipGetLastError();
-}
-
-template <int N>
-static hipError_t sob_n(int rm, bool contig, const double2* src, double2* o1, double2* o2, long long cs, int ncomp,
-                        long long inner, const double2* tw, const SobArgs& sa, const Limits& max_lds, hipStream_t s) {
-  if (rm == 8 && N > 8 && N / 8 <= 256) return sob_nr<N, 8>(contig, src, o1, o2, cs, ncomp, inner, tw, sa, max_lds, s);
-  return sob_nr<N, 16>(contig, src, o1, o2, cs, ncomp, inner, tw, sa, max_lds, s);
-}
-
-hipError_t launch_sobf(int N, int rm, bool contig, const double2* src, double2* out_sob, double2* out_lap,
-                       long long comp_stride, int ncomp, long long inner, const double2* tw, const SobArgs& sa,
-                       const Limits& max_lds, hipStream_t s) {
-  switch (N) {
-#define ATUS_CASE(n) \
-  case n: return sob_n<n>(rm, contig, src, out_sob, out_lap, comp_stride, ncomp, inner, tw, sa, max_lds, s);
-    ATUS_CASE(2) ATUS_CASE(4) ATUS_CASE(8) ATUS_CASE(16) ATUS_CASE(32) ATUS_CASE(64) ATUS_CASE(128)
-    ATUS_CASE(256) ATUS_CASE(512) ATUS_CASE(1024) ATUS_CASE(2048) ATUS_CASE(4096)
-#undef ATUS_CASE
-    default: return hipErrorInvalidValue;
-  }
-}
-
 // The passes of an iteration hold two spectra per thread, so they take the
 // plan of 8 values wherever the contiguous pencil fits a workgroup with it.
 template <int N>

@@ -14,8 +14,6 @@
 //              in one thread)
 //   k_vfuse  : inverse DFT along the last (contiguous) axis, pointwise
 //              potential / Bragg step, forward DFT along the same axis
-//   k_sobf   : forward DFT along axis 0, multiply by 1/(1+alpha k^2) and
-//              -alpha k^2, two inverse DFTs (Sobolev psi and Laplacian)
 //   k_point  : standalone pointwise steps
 //   k_reduce : deterministic two-stage reductions
 #pragma once
@@ -1165,88 +1163,36 @@ __global__ __launch_bounds__(256) void k_fs_col(double2* __restrict__ psi, long 
   }
 }
 
-// ------------------------------------------------------------ k_sobf
-// Sobolev filters along axis 0 (CSOB_Base.h:251-301 fused): from the
-// transform F of psi along the other axes, writes
-//   out_sob = inverse0( op(k) * forward0(F) ) * scale,  op = 1/(1+alpha|k|^2)
-//   out_lap = inverse0( -alpha|k|^2 * forward0(F) ) * scale  (if non-NULL)
-// k is the native-order wave vector (cft_3d.cpp:145-166).
-struct SobArgs {
-  double alpha;
-  double dk[3];
-  int n[3];
-  int dim;
-  double scale;
-};
-
+// wave number of index i of an axis of n points (a power of two), native order
 __device__ __forceinline__ double kval(int i, int n, double dk) {
   const int s = n / 2;
-  return dk * (double)(((i + s) % n) - s);
-}
-
-template <int N, int RM, bool CONTIG>
-__global__ __launch_bounds__(256) void k_sobf(const double2* src, double2* out_sob, double2* out_lap, long long comp_stride, AxisGeo g,
-                                              const double2* __restrict__ tw, SobArgs sa) {
-  extern __shared__ double2 lds_all[];
-  constexpr int R = Plan<N, RM>::R, P = Plan<N, RM>::P;
-  constexpr bool WAVE = CONTIG && (P <= 64);
-  PencilMap<N, RM, CONTIG> m(g);
-  double2* lds = lds_all + m.p * g.ls;
-  const double2* twl = stage_table<N>(lds_all + (size_t)g.T * g.ls, fft_tw<N, RM>(tw));
-  const long long coff = (long long)blockIdx.y * comp_stride;
-  double k12 = 0.0;  // sum over axes 1, 2 of k^2 (k.scale(alpha).k with isotropic alpha)
-  if constexpr (!CONTIG) {
-    const long long col = m.pid % g.inner;
-    if (sa.dim >= 2) {
-      const int i1 = (sa.dim == 3) ? (int)(col / sa.n[2]) : (int)col;
-      const double k1 = kval(i1, sa.n[1], sa.dk[1]);
-      k12 += (k1 * sa.alpha) * k1;
-    }
-    if (sa.dim == 3) {
-      const int i2 = (int)(col % sa.n[2]);
-      const double k2 = kval(i2, sa.n[2], sa.dk[2]);
-      k12 += (k2 * sa.alpha) * k2;
-    }
-  }
-  double2 v[R];
-  load_pencil<N, RM>(v, src + coff, m.base, m.stride, m.t, m.valid);
-  if constexpr (tables_in_lds<N>()) __syncthreads();
-  fft_pencil<N, RM, -1, WAVE>(v, m.t, lds, twl);
-  double2 w[R];
-#pragma unroll
-  for (int i = 0; i < R; ++i) {
-    const double k0 = kval(m.t + P * i, N, sa.dk[0]);
-    const double phi = (k0 * sa.alpha) * k0 + k12;
-    w[i] = cscale(v[i], -phi * sa.scale);
-    v[i] = cscale(v[i], sa.scale / (1.0 + phi));
-  }
-  fft_pencil<N, RM, +1, WAVE>(v, m.t, lds, twl);
-  store_pencil<N, RM>(v, out_sob + coff, m.base, m.stride, m.t, m.valid);
-  if (out_lap) {
-    fft_pencil<N, RM, +1, WAVE>(w, m.t, lds, twl);
-    store_pencil<N, RM>(w, out_lap + coff, m.base, m.stride, m.t, m.valid);
-  }
+  return dk * (double)(((i + s) & (n - 1)) - s);
 }
 
 // ------------------------------------------------------------ pointwise
 
+// indices of point l (every axis is a power of two: shifts, where 64-bit
+// divisions would bound the pointwise passes and reductions)
+__device__ __forceinline__ void split_point(long long l, const Grid& gr, int (&i)[3]) {
+  const int b2 = __ffs(gr.n[2]) - 1, b1 = __ffs(gr.n[1]) - 1;
+  i[2] = (int)l & (gr.n[2] - 1);
+  i[1] = (int)(l >> b2) & (gr.n[1] - 1);
+  i[0] = (int)(l >> (b2 + b1));
+}
+
 __device__ __forceinline__ double x0_of(long long l, const Grid& gr) {
-  const long long inner = gr.npts / gr.n[0];
-  const int i0 = (int)(l / inner);
-  return (double)(i0 - gr.n[0] / 2) * gr.dx[0];
+  int i[3];
+  split_point(l, gr, i);
+  return (double)(i[0] - gr.n[0] / 2) * gr.dx[0];
 }
 
 // beta.x over the grid's axes, summed as CPoint::operator* does
 // (CPoint.h:145-151)
 __device__ __forceinline__ double beta_dot_x(long long l, const Grid& gr, const double (&beta)[3]) {
-  long long rest = l;
-  long long idx[3] = {0, 0, 0};
-  for (int a = gr.dim - 1; a >= 0; --a) {
-    idx[a] = rest % gr.n[a];
-    rest /= gr.n[a];
-  }
+  int i[3];
+  split_point(l, gr, i);
   double bx = 0.0;
-  for (int a = 0; a < gr.dim; ++a) bx += beta[a] * ((double)(idx[a] - gr.n[a] / 2) * gr.dx[a]);
+  for (int a = 0; a < gr.dim; ++a) bx += beta[a] * ((double)(i[a] - gr.n[a] / 2) * gr.dx[a]);
   return bx;
 }
 
@@ -1377,10 +1323,9 @@ struct RedX {
   __device__ void operator()(long long l, double (&acc)[3]) const {
     const double2 a = psi[l];
     const double d = a.x * a.x + a.y * a.y;
-    const long long n12 = (long long)gr.n[1] * gr.n[2];
-    const int i0 = (int)(l / n12);
-    const int i1 = (int)((l - i0 * n12) / gr.n[2]);
-    const int i2 = (int)(l - i0 * n12 - (long long)i1 * gr.n[2]);
+    int id[3];
+    split_point(l, gr, id);
+    const int i0 = id[0], i1 = id[1], i2 = id[2];
     acc[0] += ((double)(i0 - gr.n[0] / 2) * gr.dx[0]) * d;
     acc[1] += ((double)(i1 - gr.n[1] / 2) * gr.dx[1]) * d;
     acc[2] += ((double)(i2 - gr.n[2] / 2) * gr.dx[2]) * d;
@@ -1388,10 +1333,9 @@ struct RedX {
 };
 
 __device__ __forceinline__ void k_of(long long l, const Grid& gr, double (&k)[3]) {
-  const long long n12 = (long long)gr.n[1] * gr.n[2];
-  const int i0 = (int)(l / n12);
-  const int i1 = (int)((l - i0 * n12) / gr.n[2]);
-  const int i2 = (int)(l - i0 * n12 - (long long)i1 * gr.n[2]);
+  int id[3];
+  split_point(l, gr, id);
+  const int i0 = id[0], i1 = id[1], i2 = id[2];
   k[0] = kval(i0, gr.n[0], gr.dk[0]);
   k[1] = gr.dim > 1 ? kval(i1, gr.n[1], gr.dk[1]) : 0.0;
   k[2] = gr.dim > 2 ? kval(i2, gr.n[2], gr.dk[2]) : 0.0;
@@ -1422,10 +1366,9 @@ struct RedMom1 {
   __device__ void operator()(long long l, double (&acc)[5]) const {
     const double2 a = psi[l];
     const double d = a.x * a.x + a.y * a.y;
-    const long long n12 = (long long)gr.n[1] * gr.n[2];
-    const int i0 = (int)(l / n12);
-    const int i1 = (int)((l - i0 * n12) / gr.n[2]);
-    const int i2 = (int)(l - i0 * n12 - (long long)i1 * gr.n[2]);
+    int id[3];
+    split_point(l, gr, id);
+    const int i0 = id[0], i1 = id[1], i2 = id[2];
     acc[0] += d;
     acc[1] += ((double)(i0 - gr.n[0] / 2) * gr.dx[0]) * d;
     acc[2] += ((double)(i1 - gr.n[1] / 2) * gr.dx[1]) * d;
@@ -1445,11 +1388,8 @@ struct RedMom2 {
   __device__ void operator()(long long l, double (&acc)[3]) const {
     const double2 a = psi[l];
     const double d = a.x * a.x + a.y * a.y;
-    const long long n12 = (long long)gr.n[1] * gr.n[2];
-    const int i0 = (int)(l / n12);
-    const int i1 = (int)((l - i0 * n12) / gr.n[2]);
-    const int i2 = (int)(l - i0 * n12 - (long long)i1 * gr.n[2]);
-    const int id[3] = {i0, i1, i2};
+    int id[3];
+    split_point(l, gr, id);
 #pragma unroll
     for (int ax = 0; ax < 3; ++ax) {
       const double c = KSPACE ? kval(id[ax], gr.n[ax], gr.dk[ax]) : (double)(id[ax] - gr.n[ax] / 2) * gr.dx[ax];
@@ -1665,24 +1605,27 @@ struct RedEkin {
 };
 
 // potential + interaction energy sum_i (V_i + 1/2 sum_j g_ij n_j) n_i
+template <int NC>
 struct RedEpot {
   static constexpr int NV = 1;
   const double2* psi;
   const double* pot;
   long long npts;
-  int nc;
   double gs[16];
   __device__ void operator()(long long l, double (&acc)[1]) const {
-    double n[4];
-    for (int i = 0; i < nc; ++i) {
+    double n[NC];
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
       const double2 a = psi[i * npts + l];
       n[i] = a.x * a.x + a.y * a.y;
     }
     double e = 0.0;
-    for (int i = 0; i < nc; ++i) {
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
       const double v = pot ? pot[i * npts + l] : 0.0;
       double nl = 0.0;
-      for (int j = 0; j < nc; ++j) nl += gs[j + nc * i] * n[j];
+#pragma unroll
+      for (int j = 0; j < NC; ++j) nl += gs[j + NC * i] * n[j];
       e += (v + 0.5 * nl) * n[i];
     }
     acc[0] += e;

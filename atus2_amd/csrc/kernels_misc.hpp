@@ -10,11 +10,10 @@ namespace atus {
 __global__ __launch_bounds__(256) void k_momentum(double2* __restrict__ psi, Grid gr, double p0, double p1,
                                                   double p2) {
   const long long stride = (long long)gridDim.x * blockDim.x;
-  const long long n12 = (long long)gr.n[1] * gr.n[2];
   for (long long l = (long long)blockIdx.x * blockDim.x + threadIdx.x; l < gr.npts; l += stride) {
-    const int i0 = (int)(l / n12);
-    const int i1 = (int)((l - i0 * n12) / gr.n[2]);
-    const int i2 = (int)(l - i0 * n12 - (long long)i1 * gr.n[2]);
+    int id[3];
+    split_point(l, gr, id);
+    const int i0 = id[0], i1 = id[1], i2 = id[2];
     double px = p0 * ((double)(i0 - gr.n[0] / 2) * gr.dx[0]);
     if (gr.dim > 1) px += p1 * ((double)(i1 - gr.n[1] / 2) * gr.dx[1]);
     if (gr.dim > 2) px += p2 * ((double)(i2 - gr.n[2] / 2) * gr.dx[2]);
@@ -22,23 +21,6 @@ __global__ __launch_bounds__(256) void k_momentum(double2* __restrict__ psi, Gri
     sincos(px, &s, &c);
     const double2 a = psi[l];
     psi[l] = make_double2(a.x * c - a.y * s, a.x * s + a.y * c);
-  }
-}
-
-// multiply a component by a complex table per point (kinetic step of the
-// unfused path)
-__global__ __launch_bounds__(256) void k_mul_phase(double2* __restrict__ psi, long long npts, KinTabs kt, int n1,
-                                                   int n2, int dim) {
-  const long long stride = (long long)gridDim.x * blockDim.x;
-  const long long n12 = (long long)n1 * n2;
-  for (long long l = (long long)blockIdx.x * blockDim.x + threadIdx.x; l < npts; l += stride) {
-    const int i0 = (int)(l / n12);
-    const int i1 = (int)((l - i0 * n12) / n2);
-    const int i2 = (int)(l - i0 * n12 - (long long)i1 * n2);
-    double2 e = kt.e0[i0];
-    if (dim > 1) e = cmul(e, kt.e1[i1]);
-    if (dim > 2) e = cmul(e, kt.e2[i2]);
-    psi[blockIdx.y * npts + l] = cmul(psi[blockIdx.y * npts + l], e);
   }
 }
 
@@ -55,12 +37,8 @@ __global__ __launch_bounds__(256) void k_inflate(const double2* __restrict__ src
   const double2* s = src + (long long)blockIdx.y * src_stride;
   double2* d = dst + (long long)blockIdx.y * dst_stride;
   for (long long l = (long long)blockIdx.x * blockDim.x + threadIdx.x; l < gd.npts; l += stride) {
-    long long rest = l;
-    int id[3] = {0, 0, 0};
-    for (int a = 2; a >= 0; --a) {
-      id[a] = (int)(rest % gd.n[a]);
-      rest /= gd.n[a];
-    }
+    int id[3];
+    split_point(l, gd, id);
     bool inside = true;
     long long ls = 0;
     for (int a = 0; a < 3; ++a) {

@@ -159,10 +159,12 @@ hipError_t launch_rabi_box(int axis, int rm, const double2* src, long long seg, 
                            const double2* tw, const RabiBox& rb, const Limits& lim, double* partials,
                            unsigned* nblocks, hipStream_t s);
 
-// Sobolev filters along axis 0
-hipError_t launch_sobf(int N, int rm, bool contig, const double2* src, double2* out_sob, double2* out_lap,
-                       long long comp_stride, int ncomp, long long inner, const double2* tw, const SobArgs& sa,
-                       const Limits& max_lds, hipStream_t s);
+// densities along one axis of N points (k_marginal): out[j] the sums of
+// |psi|^2 and of |F psi|^2 over the others, through part [*nblocks][N];
+// phase (contiguous axis only, or NULL) [*nblocks]; part NULL: only *nblocks
+hipError_t launch_marginal(int N, const double2* psi, long long inner, long long outer, const double2* tw,
+                           double2* part, double2* out, double* phase, unsigned* nblocks, const Limits& lim,
+                           hipStream_t s);
 
 // the passes of a Sobolev iteration on a 2D/3D grid of nw (1 or 2) wave
 // functions (sob.hpp); partials NULL: only *nblocks,
