@@ -4,6 +4,7 @@
 // and Adam moments are fp32; matrix-product operands are rounded to bf16.
 // No counterpart in the reference: the network only proposes the start
 // state that CSOB_Base's iteration then polishes.
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include <vector>
@@ -27,13 +28,17 @@ struct atus_net {
   float* t = nullptr;                                           // targets
   float* work = nullptr;
   size_t work_floats = 0;
-  float* part = nullptr;
-  std::vector<float> part_host;
-  int nblk = 256;
+  float* part = nullptr;  // loss partials of a batch
+  float* loss = nullptr;  // [CHUNK] losses of the steps in flight
+  int* bad = nullptr;     // a loss was not finite (mlp_loss)
   float* data_x = nullptr;
   float* data_t = nullptr;
   int ndata = 0;
+  // training steps enqueued between two synchronisations, and the rows of
+  // their batches
+  static constexpr int CHUNK = 256;
   int* idx = nullptr;
+  int idx_cap = 0;
   long long step = 0;
   bool split = true;  // matrix products as hi/lo bf16 pairs (atus_net_set_precision)
 };
@@ -54,44 +59,57 @@ int check_net(atus_net* n) {
   return hipSetDevice(n->device) == hipSuccess ? ATUS_OK : fail(ATUS_ERR_HIP, "hipSetDevice failed");
 }
 
-int forward(atus_net* n, int B) {
+// activations of a batch.  T: the last layer forms the gradient of the mean
+// squared error of its output against T (rows idx, or 0..B-1) in d[4]
+// instead of the output, and the loss partials
+int forward(atus_net* n, int B, const float* T = nullptr, const int* idx = nullptr) {
   for (int l = 0; l < 4; ++l) {
     const int in = n->dims[l], out = n->dims[l + 1];
-    HIP_TRY(mlp_gemm(n->x[l], in, 1, n->p + n->off_w[l], out, 1, n->x[l + 1], B, out, in, n->p + n->off_b[l],
-                     l < 3 ? 1 : 0, n->work, n->work_floats, n->stream, n->split));
+    GemmEpilogue e;
+    e.bias = n->p + n->off_b[l];
+    e.act = l < 3 ? 1 : 0;
+    const bool mse = l == 3 && T;
+    if (mse) {
+      e.T = T;
+      e.idx = idx;
+      e.scale = 2.f / (float)((long long)B * out);
+      e.loss = n->part;
+    }
+    HIP_TRY(mlp_gemm(n->x[l], in, 1, n->p + n->off_w[l], out, 1, mse ? n->d[4] : n->x[l + 1], B, out, in, e, n->work,
+                     n->work_floats, n->stream, n->split));
   }
   return ATUS_OK;
 }
 
-// gradients of the mean squared error of x[4] against t into n->g; loss
-int backward(atus_net* n, int B, double* loss) {
-  const long long ny = (long long)B * n->dims[4];
-  HIP_TRY(mlp_mse(n->x[4], n->t, ny, n->d[4], n->part, n->nblk, n->stream));
+// from d[4]: the parameters' gradients into n->g, and the loss into
+// n->loss[slot]
+int backward(atus_net* n, int B, int slot) {
+  HIP_TRY(mlp_loss(n->part, (int)mlp_loss_parts(B, n->dims[4]), (double)B * n->dims[4], n->loss, slot, n->bad,
+                   n->stream));
   for (int l = 3; l >= 0; --l) {
     const int in = n->dims[l], out = n->dims[l + 1];
-    float* dz = n->d[l + 1];
-    if (l < 3) HIP_TRY(mlp_tanh_back(dz, n->x[l + 1], dz, (long long)B * out, n->stream));
-    // dW = x^T dZ, db = column sums of dZ, dX = dZ W^T
-    HIP_TRY(mlp_gemm(n->x[l], 1, in, dz, out, 1, n->g + n->off_w[l], in, out, B, nullptr, 0, n->work,
-                     n->work_floats, n->stream, n->split));
-    HIP_TRY(mlp_colsum(dz, B, out, n->g + n->off_b[l], n->stream));
-    if (l > 0)
-      HIP_TRY(mlp_gemm(dz, out, 1, n->p + n->off_w[l], 1, out, n->d[l], B, in, out, nullptr, 0, n->work,
-                       n->work_floats, n->stream, n->split));
+    const float* dz = n->d[l + 1];
+    // dW = x^T dZ, db = column sums of dZ
+    GemmEpilogue w;
+    w.colsum = n->g + n->off_b[l];
+    HIP_TRY(mlp_gemm(n->x[l], 1, in, dz, out, 1, n->g + n->off_w[l], in, out, B, w, n->work, n->work_floats, n->stream,
+                     n->split));
+    if (l > 0) {
+      // the next layer's dZ = (dZ W^T) (1 - x^2)
+      GemmEpilogue e;
+      e.act = 2;
+      e.X = n->x[l];
+      HIP_TRY(mlp_gemm(dz, out, 1, n->p + n->off_w[l], 1, out, n->d[l], B, in, out, e, n->work, n->work_floats,
+                       n->stream, n->split));
+    }
   }
-  HIP_TRY(hipMemcpyAsync(n->part_host.data(), n->part, sizeof(float) * n->nblk, hipMemcpyDeviceToHost, n->stream));
-  HIP_TRY(hipStreamSynchronize(n->stream));
-  double s = 0.0;
-  for (int b = 0; b < n->nblk; ++b) s += n->part_host[b];
-  *loss = s / (double)ny;
   return ATUS_OK;
 }
 
-int adam_step(atus_net* n, float lr) {
+int adam_step(atus_net* n, long long step, float lr) {
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
-  ++n->step;
-  const float c1 = 1.f - powf(b1, (float)n->step), c2 = 1.f - powf(b2, (float)n->step);
-  HIP_TRY(mlp_adam(n->p, n->g, n->m, n->v, n->np, lr, b1, b2, eps, c1, c2, n->stream));
+  const float c1 = 1.f - powf(b1, (float)step), c2 = 1.f - powf(b2, (float)step);
+  HIP_TRY(mlp_adam(n->p, n->g, n->m, n->v, n->np, lr, b1, b2, eps, c1, c2, n->bad, n->stream));
   return ATUS_OK;
 }
 
@@ -138,13 +156,15 @@ int atus_net_create(atus_net** out, int n_in, int h1, int h2, int h3, int n_out,
     work = std::max(work, mlp_gemm_work(max_batch, in, o));  // dX
   }
   n->work_floats = work;
-  n->part_host.resize(n->nblk);
+  n->idx_cap = std::max(65536, max_batch);
   bool ok = hipMalloc(&n->p, sizeof(float) * n->np) == hipSuccess && hipMalloc(&n->g, sizeof(float) * n->np) == hipSuccess &&
             hipMalloc(&n->m, sizeof(float) * n->np) == hipSuccess && hipMalloc(&n->v, sizeof(float) * n->np) == hipSuccess &&
-            hipMalloc(&n->work, sizeof(float) * work) == hipSuccess &&
-            hipMalloc(&n->part, sizeof(float) * n->nblk) == hipSuccess &&
+            hipMalloc(&n->work, sizeof(float) * std::max<size_t>(work, 1)) == hipSuccess &&
+            hipMalloc(&n->part, sizeof(float) * mlp_loss_parts(max_batch, n_out)) == hipSuccess &&
+            hipMalloc(&n->loss, sizeof(float) * atus_net::CHUNK) == hipSuccess &&
+            hipMalloc(&n->bad, sizeof(int)) == hipSuccess &&
             hipMalloc(&n->t, sizeof(float) * (size_t)max_batch * n_out) == hipSuccess &&
-            hipMalloc(&n->idx, sizeof(int) * max_batch) == hipSuccess;
+            hipMalloc(&n->idx, sizeof(int) * n->idx_cap) == hipSuccess;
   for (int l = 0; ok && l < 5; ++l) {
     ok = hipMalloc(&n->x[l], sizeof(float) * (size_t)max_batch * dims[l]) == hipSuccess;
     if (ok && l > 0) ok = hipMalloc(&n->d[l], sizeof(float) * (size_t)max_batch * dims[l]) == hipSuccess;
@@ -169,12 +189,13 @@ int atus_net_destroy(atus_net* n) {
   if (!n) return ATUS_OK;
   (void)hipSetDevice(n->device);
   if (n->stream) (void)hipStreamSynchronize(n->stream);
-  for (float* q : {n->p, n->g, n->m, n->v, n->work, n->part, n->t, n->data_x, n->data_t}) (void)hipFree(q);
+  for (float* q : {n->p, n->g, n->m, n->v, n->work, n->part, n->loss, n->t, n->data_x, n->data_t}) (void)hipFree(q);
   for (int l = 0; l < 5; ++l) {
     (void)hipFree(n->x[l]);
     (void)hipFree(n->d[l]);
   }
   (void)hipFree(n->idx);
+  (void)hipFree(n->bad);
   if (n->stream) (void)hipStreamDestroy(n->stream);
   delete n;
   return ATUS_OK;
@@ -232,14 +253,11 @@ int atus_net_gradients(atus_net* n, const float* x, const float* t, int batch, f
   if (!x || !t || !loss) return fail(ATUS_ERR_ARG, "null argument");
   HIP_TRY(hipMemcpyAsync(n->x[0], x, sizeof(float) * batch * n->dims[0], hipMemcpyHostToDevice, n->stream));
   HIP_TRY(hipMemcpyAsync(n->t, t, sizeof(float) * (size_t)batch * n->dims[4], hipMemcpyHostToDevice, n->stream));
-  ATUS_TRY(forward(n, batch));
-  double l = 0.0;
-  ATUS_TRY(backward(n, batch, &l));
-  *loss = (float)l;
-  if (grads) {
-    HIP_TRY(hipMemcpyAsync(grads, n->g, sizeof(float) * n->np, hipMemcpyDeviceToHost, n->stream));
-    HIP_TRY(hipStreamSynchronize(n->stream));
-  }
+  ATUS_TRY(forward(n, batch, n->t));
+  ATUS_TRY(backward(n, batch, 0));
+  HIP_TRY(hipMemcpyAsync(loss, n->loss, sizeof(float), hipMemcpyDeviceToHost, n->stream));
+  if (grads) HIP_TRY(hipMemcpyAsync(grads, n->g, sizeof(float) * n->np, hipMemcpyDeviceToHost, n->stream));
+  HIP_TRY(hipStreamSynchronize(n->stream));
   return ATUS_OK;
 }
 
@@ -271,25 +289,42 @@ int atus_net_train(atus_net* n, int steps, int batch, float lr, float lr_final, 
   for (int i = 0; i < n->ndata; ++i) perm[i] = i;
   uint64_t s = seed;
   int pos = n->ndata;  // reshuffle before the first batch
-  for (int it = 0; it < steps; ++it) {
-    if (pos + batch > n->ndata) {
-      for (int i = n->ndata - 1; i > 0; --i) std::swap(perm[i], perm[(int)(splitmix64(s) % (uint64_t)(i + 1))]);
-      pos = 0;
+  HIP_TRY(hipMemsetAsync(n->bad, 0, sizeof(int), n->stream));
+  // chunks of steps without a host round trip: their batches' rows go up
+  // first, their losses come back last
+  const int chunk = std::min(atus_net::CHUNK, n->idx_cap / batch);
+  std::vector<int> rows((size_t)chunk * batch);
+  std::vector<float> got(chunk);
+  for (int it0 = 0; it0 < steps; it0 += chunk) {
+    const int m = std::min(chunk, steps - it0);
+    for (int k = 0; k < m; ++k) {
+      if (pos + batch > n->ndata) {
+        for (int i = n->ndata - 1; i > 0; --i) std::swap(perm[i], perm[(int)(splitmix64(s) % (uint64_t)(i + 1))]);
+        pos = 0;
+      }
+      std::copy(perm.begin() + pos, perm.begin() + pos + batch, rows.begin() + (size_t)k * batch);
+      pos += batch;
     }
-    HIP_TRY(hipMemcpyAsync(n->idx, perm.data() + pos, sizeof(int) * batch, hipMemcpyHostToDevice, n->stream));
-    pos += batch;
-    HIP_TRY(mlp_gather(n->data_x, n->idx, batch, n->dims[0], n->x[0], n->stream));
-    HIP_TRY(mlp_gather(n->data_t, n->idx, batch, n->dims[4], n->t, n->stream));
-    ATUS_TRY(forward(n, batch));
-    double l = 0.0;
-    ATUS_TRY(backward(n, batch, &l));
-    if (!std::isfinite(l)) return fail(ATUS_ERR_NUMERIC, "training loss is not finite");
-    if (losses) losses[it] = (float)l;
-    // cosine decay from lr to lr_final
-    const double c = 0.5 * (1.0 + cos(M_PI * (double)it / (double)steps));
-    ATUS_TRY(adam_step(n, (float)(lr_final + (lr - lr_final) * c)));
+    HIP_TRY(hipMemcpyAsync(n->idx, rows.data(), sizeof(int) * (size_t)m * batch, hipMemcpyHostToDevice, n->stream));
+    for (int k = 0; k < m; ++k) {
+      const int* idx = n->idx + (size_t)k * batch;
+      HIP_TRY(mlp_gather(n->data_x, idx, batch, n->dims[0], n->x[0], n->stream));
+      ATUS_TRY(forward(n, batch, n->data_t, idx));
+      ATUS_TRY(backward(n, batch, k));
+      // cosine decay from lr to lr_final
+      const double c = 0.5 * (1.0 + cos(M_PI * (double)(it0 + k) / (double)steps));
+      ATUS_TRY(adam_step(n, n->step + k + 1, (float)(lr_final + (lr - lr_final) * c)));
+    }
+    HIP_TRY(hipMemcpyAsync(got.data(), n->loss, sizeof(float) * m, hipMemcpyDeviceToHost, n->stream));
+    HIP_TRY(hipStreamSynchronize(n->stream));
+    for (int k = 0; k < m; ++k) {
+      // from the first loss that is not finite on, Adam has left the
+      // parameters alone
+      if (!std::isfinite(got[k])) return fail(ATUS_ERR_NUMERIC, "training loss is not finite");
+      if (losses) losses[it0 + k] = got[k];
+      ++n->step;
+    }
   }
-  HIP_TRY(hipStreamSynchronize(n->stream));
   return ATUS_OK;
 }
 

@@ -2,6 +2,7 @@
 // products with FP32 accumulation (v_mfma_f32_16x16x32_bf16), their
 // epilogues, the loss, the optimiser, and the separable interpolation of
 // the network's 32^3 output onto a solver grid.
+#include "launch.hpp"
 #include "mlp.hpp"
 
 namespace atus {
@@ -9,108 +10,216 @@ namespace atus {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-// P[z][m][n] = sum over k in [z*kchunk, (z+1)*kchunk) of A(m,k) B(k,n), with
-// A(m,k) = A[m*sam + k*sak] and B(k,n) = B[k*sbk + n*sbn] rounded to bf16
-// (SPLIT false), or split as a = hi + lo, hi = bf16(a), lo = bf16(a - hi),
-// with a b ~ hi_a hi_b + hi_a lo_b + lo_a hi_b (SPLIT true: three products
-// per slice, about 16 significant bits per operand).
-// One wavefront per 16x16 tile; lane l holds A rows l%16 and B columns
-// l%16 at k = 8*(l/16) + 0..7 of each 32-wide slice, and receives rows
-// 4*(l/16) + 0..3 of column l%16 of the tile.
-template <bool SPLIT>
-__global__ __launch_bounds__(64) void k_gemm_bf16(const float* __restrict__ A, long long sam, long long sak,
-                                                  const float* __restrict__ B, long long sbk, long long sbn,
-                                                  float* __restrict__ P, int M, int N, int K, int kchunk) {
-  const int lane = threadIdx.x;
-  const int n0 = blockIdx.x * 16, m0 = blockIdx.y * 16;
-  const int kb = blockIdx.z * kchunk;
-  const int ke = min(K, kb + kchunk);
-  const int i = lane & 15, grp = lane >> 4;
-  const int m = m0 + i, n = n0 + i;
-  const bool mok = m < M, nok = n < N;
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  for (int k0 = kb; k0 < ke; k0 += 32) {
-    bf16x8 a, b, al, bl;
+// ---------------------------------------------------------------- products
+// C(m,n) = sum_k A(m,k) B(k,n), A(m,k) = A[m*sam + k*sak], B(k,n) =
+// B[k*sbk + n*sbn], operands rounded to bf16 (SPLIT false) or split as a = hi
+// + lo, hi = bf16(a), lo = bf16(a - hi), with a b ~ hi_a hi_b + hi_a lo_b +
+// lo_a hi_b (SPLIT true: three products, about 16 significant bits per
+// operand), fp32 accumulation.
+//
+// A workgroup of four wavefronts forms a 64 x 64 tile in slices of 32 along
+// k.  An operand's slice goes through LDS as [row][k], 8 consecutive k of a
+// row per 16-byte write, so each element is read from memory and split once
+// per tile instead of once per 16 x 16 tile and wavefront; the next slice is
+// in flight in registers while this one is multiplied.  The large products
+// (256 x 32768 x 64 and its two transposes) stream their operands; what
+// follows them rides in their epilogues rather than in passes of its own.
+constexpr int GT = 64;        // tile edge
+constexpr int GK = 32;        // slice along k
+constexpr int GP = GK + 8;    // LDS row pitch: 16-byte rows on distinct banks
+
+enum GemmMode {
+  G_OUT = 0,    // C = act(sum + bias)
+  G_PART = 1,   // P[blockIdx.z][m][n]: partial sums of a split along k
+  G_MSE = 2     // d = sum + bias - T[row(m)][n]: C = 2 d / count, loss partials
+};
+
+struct GemmArgs {
+  const float* A;
+  long long sam, sak;
+  const float* B;
+  long long sbk, sbn;
+  float* C;
+  int M, N, K, kchunk;
+  int mode;
+  GemmEpilogue e;
+};
+
+// 8 values of an operand's row r at k0..k0+7 (0 beyond the matrix)
+__device__ __forceinline__ void gemm_load(float (&f)[8], const float* src, long long sr, long long sk, int r, int rows,
+                                          int k0, int ke, bool vec) {
+  const float* p = src + (long long)r * sr + (long long)k0 * sk;
+  if (vec && r < rows && k0 + 8 <= ke) {
+    const float4 x = *reinterpret_cast<const float4*>(p), y = *reinterpret_cast<const float4*>(p + 4);
+    f[0] = x.x, f[1] = x.y, f[2] = x.z, f[3] = x.w;
+    f[4] = y.x, f[5] = y.y, f[6] = y.z, f[7] = y.w;
+  } else {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int k = k0 + 8 * grp + j;
-      const bool kin = k < ke;
-      const float fa = (kin && mok) ? A[(long long)m * sam + (long long)k * sak] : 0.f;
-      const float fb = (kin && nok) ? B[(long long)k * sbk + (long long)n * sbn] : 0.f;
-      a[j] = (__bf16)fa;
-      b[j] = (__bf16)fb;
-      if constexpr (SPLIT) {
-        al[j] = (__bf16)(fa - (float)a[j]);
-        bl[j] = (__bf16)(fb - (float)b[j]);
-      }
-    }
-    if constexpr (SPLIT) {
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, b, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bl, acc, 0, 0, 0);
-    }
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
-  }
-  float* out = P + (long long)blockIdx.z * M * N;
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int row = m0 + 4 * grp + r, col = n0 + i;
-    if (row < M && col < N) out[(long long)row * N + col] = acc[r];
+    for (int j = 0; j < 8; ++j) f[j] = (r < rows && k0 + j < ke) ? p[(long long)j * sk] : 0.f;
   }
 }
 
-// C[m][n] = act(sum_z P[z][m][n] + bias[n]); act 1: tanh.  Split order fixed.
+template <bool SPLIT>
+__device__ __forceinline__ void gemm_store(const float (&f)[8], __bf16* hi, __bf16* lo, int at) {
+  bf16x8 h, l;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    h[j] = (__bf16)f[j];
+    if constexpr (SPLIT) l[j] = (__bf16)(f[j] - (float)h[j]);
+  }
+  *reinterpret_cast<bf16x8*>(hi + at) = h;
+  if constexpr (SPLIT) *reinterpret_cast<bf16x8*>(lo + at) = l;
+}
+
+__device__ __forceinline__ float gemm_act(float s, int act, const float* X, long long at) {
+  if (act == 1) return tanhf(s);
+  if (act == 2) return s * (1.f - X[at] * X[at]);  // dZ = dX (1 - X^2), X = tanh(Z)
+  return s;
+}
+
+template <bool SPLIT>
+__global__ __launch_bounds__(256) void k_gemm_bf16(GemmArgs g) {
+  __shared__ __attribute__((aligned(16))) __bf16 sh[SPLIT ? 4 : 2][GT * GP];
+  __shared__ float red[256];
+  __bf16* ah = sh[0];
+  __bf16* bh = sh[1];
+  __bf16* al = sh[SPLIT ? 2 : 0];
+  __bf16* bl = sh[SPLIT ? 3 : 1];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int n0 = blockIdx.x * GT, m0 = blockIdx.y * GT;
+  const int kb = blockIdx.z * g.kchunk, ke = min(g.K, kb + g.kchunk);
+  // this thread's share of a slice: 8 k of one row of each operand.  Rows
+  // run over the lanes where the operand is contiguous along them, k
+  // groups where it is contiguous along k.
+  const bool ak = g.sak == 1, bk = g.sbk == 1;
+  const int ar = ak ? tid >> 2 : tid & 63, ag = ak ? tid & 3 : tid >> 6;
+  const int br = bk ? tid >> 2 : tid & 63, bg = bk ? tid & 3 : tid >> 6;
+  const bool av = ak && (g.sam & 3) == 0 && ((unsigned long long)g.A & 15) == 0;
+  const bool bv = bk && (g.sbn & 3) == 0 && ((unsigned long long)g.B & 15) == 0;
+  float fa[8], fb[8], bsum = 0.f;
+  f32x4 acc[2][2] = {};
+  const int i = lane & 15, grp = lane >> 4;
+  const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
+  gemm_load(fa, g.A, g.sam, g.sak, m0 + ar, g.M, kb + 8 * ag, ke, av);
+  gemm_load(fb, g.B, g.sbn, g.sbk, n0 + br, g.N, kb + 8 * bg, ke, bv);
+  for (int k0 = kb; k0 < ke; k0 += GK) {
+    __syncthreads();  // the last slice's reads are done
+    gemm_store<SPLIT>(fa, ah, al, ar * GP + 8 * ag);
+    gemm_store<SPLIT>(fb, bh, bl, br * GP + 8 * bg);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) bsum += fb[j];
+    __syncthreads();
+    if (k0 + GK < ke) {
+      gemm_load(fa, g.A, g.sam, g.sak, m0 + ar, g.M, k0 + GK + 8 * ag, ke, av);
+      gemm_load(fb, g.B, g.sbn, g.sbk, n0 + br, g.N, k0 + GK + 8 * bg, ke, bv);
+    }
+    bf16x8 a[2], b[2], a2[2], b2[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int oa = (wm + 16 * t + i) * GP + 8 * grp, ob = (wn + 16 * t + i) * GP + 8 * grp;
+      a[t] = *reinterpret_cast<const bf16x8*>(ah + oa);
+      b[t] = *reinterpret_cast<const bf16x8*>(bh + ob);
+      if constexpr (SPLIT) {
+        a2[t] = *reinterpret_cast<const bf16x8*>(al + oa);
+        b2[t] = *reinterpret_cast<const bf16x8*>(bl + ob);
+      }
+    }
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int y = 0; y < 2; ++y) {
+        if constexpr (SPLIT) {
+          acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2[x], b[y], acc[x][y], 0, 0, 0);
+          acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[x], b2[y], acc[x][y], 0, 0, 0);
+        }
+        acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[x], b[y], acc[x][y], 0, 0, 0);
+      }
+  }
+  // lane l holds rows 4 (l/16) + 0..3 of column l%16 of each 16 x 16 tile
+  float loss = 0.f;
+#pragma unroll
+  for (int x = 0; x < 2; ++x)
+#pragma unroll
+    for (int y = 0; y < 2; ++y)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = m0 + wm + 16 * x + 4 * grp + r, col = n0 + wn + 16 * y + i;
+        if (row >= g.M || col >= g.N) continue;
+        const long long at = (long long)row * g.N + col;
+        if (g.mode == G_PART) {
+          g.C[(long long)blockIdx.z * g.M * g.N + at] = acc[x][y][r];
+        } else {
+          float s = acc[x][y][r];
+          if (g.e.bias) s += g.e.bias[col];
+          if (g.mode == G_MSE) {
+            const float d = s - g.e.T[(long long)(g.e.idx ? g.e.idx[row] : row) * g.N + col];
+            g.C[at] = g.e.scale * d;
+            loss += d * d;
+          } else {
+            g.C[at] = gemm_act(s, g.e.act, g.e.X, at);
+          }
+        }
+      }
+  if (g.mode == G_MSE) {
+    red[tid] = loss;
+    __syncthreads();
+    for (int q = 128; q > 0; q >>= 1) {
+      if (tid < q) red[tid] += red[tid + q];
+      __syncthreads();
+    }
+    if (tid == 0) g.e.loss[blockIdx.y * gridDim.x + blockIdx.x] = red[0];
+  }
+  if (g.e.colsum && blockIdx.y == 0) {
+    // column sums of B (one slice group per wavefront or lane quad)
+    red[tid] = bsum;
+    __syncthreads();
+    if (tid < GT && n0 + tid < g.N) {
+      float s = 0.f;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) s += red[bk ? 4 * tid + q : tid + GT * q];
+      g.e.colsum[n0 + tid] = s;
+    }
+  }
+}
+
+// C[m][n] = act(sum_z P[z][m][n] + bias[n]), splits in order
 __global__ __launch_bounds__(256) void k_gemm_sum(const float* __restrict__ P, int splits, int M, int N,
-                                                  const float* __restrict__ bias, int act, float* __restrict__ C) {
+                                                  GemmEpilogue ep, float* __restrict__ C) {
   const long long MN = (long long)M * N;
   for (long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x; e < MN; e += (long long)gridDim.x * blockDim.x) {
     float s = 0.f;
     for (int z = 0; z < splits; ++z) s += P[z * MN + e];
-    if (bias) s += bias[e % N];
-    C[e] = act == 1 ? tanhf(s) : s;
+    if (ep.bias) s += ep.bias[e % N];
+    C[e] = gemm_act(s, ep.act, ep.X, e);
   }
 }
 
-// dZ = dX (1 - X^2), X = tanh(Z)
-__global__ __launch_bounds__(256) void k_tanh_back(const float* __restrict__ dX, const float* __restrict__ X,
-                                                   float* __restrict__ dZ, long long n) {
-  for (long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += (long long)gridDim.x * blockDim.x)
-    dZ[e] = dX[e] * (1.f - X[e] * X[e]);
-}
-
-// db[n] = sum_m dZ[m][n], rows in order
-__global__ __launch_bounds__(256) void k_colsum(const float* __restrict__ dZ, int M, int N, float* __restrict__ db) {
-  const int n = blockIdx.x * blockDim.x + threadIdx.x;
-  if (n >= N) return;
-  float s = 0.f;
-  for (int m = 0; m < M; ++m) s += dZ[(long long)m * N + n];
-  db[n] = s;
-}
-
-// mean squared error over n values: dY = 2 (Y - T) / n; per-block partial
-// sums of (Y - T)^2 (fixed order within and across blocks)
-__global__ __launch_bounds__(256) void k_mse(const float* __restrict__ Y, const float* __restrict__ T, long long n,
-                                             float* __restrict__ dY, float* __restrict__ part) {
-  __shared__ float sh[256];
-  float acc = 0.f;
-  const float sc = 2.f / (float)n;
-  for (long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += (long long)gridDim.x * blockDim.x) {
-    const float d = Y[e] - T[e];
-    dY[e] = sc * d;
-    acc += d * d;
-  }
+// mean squared error of step `slot`: loss[slot] = sum of the nb partials / n
+// (fixed order); a value that is not finite sets *bad, which stays set and
+// keeps Adam from changing the parameters from then on
+__global__ __launch_bounds__(256) void k_loss(const float* __restrict__ part, int nb, double n, float* __restrict__ loss,
+                                              int slot, int* __restrict__ bad) {
+  __shared__ double sh[256];
+  double acc = 0.0;
+  for (int b = threadIdx.x; b < nb; b += 256) acc += part[b];
   sh[threadIdx.x] = acc;
   __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if ((int)threadIdx.x < s) sh[threadIdx.x] += sh[threadIdx.x + s];
+  for (int q = 128; q > 0; q >>= 1) {
+    if ((int)threadIdx.x < q) sh[threadIdx.x] += sh[threadIdx.x + q];
     __syncthreads();
   }
-  if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
+  if (threadIdx.x == 0) {
+    const double l = sh[0] / n;
+    loss[slot] = (float)l;
+    if (!isfinite(l)) *bad = 1;
+  }
 }
 
 // Adam (Kingma & Ba 2015) with bias corrections c1 = 1 - beta1^t, c2 = 1 - beta2^t
 __global__ __launch_bounds__(256) void k_adam(float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m,
                                               float* __restrict__ v, long long n, float lr, float b1, float b2,
-                                              float eps, float c1, float c2) {
+                                              float eps, float c1, float c2, const int* __restrict__ bad) {
+  if (*bad) return;
   for (long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += (long long)gridDim.x * blockDim.x) {
     const float ge = g[e];
     const float me = b1 * m[e] + (1.f - b1) * ge;
@@ -164,60 +273,63 @@ static unsigned ew_grid(long long n) {
   return (unsigned)b;
 }
 
-// split of K into 32-wide slices so that tiles x splits is about 2048
+// Split of K: products of fewer tiles than CUs and more than 8 slices give
+// every CU a tile of at least 8 slices of its own (256 x 64 x 32768: 64
+// splits of 16 slices, 256 workgroups); shorter ones are not worth the second launch
 static void split_plan(int M, int N, int K, int* splits, int* kchunk) {
-  const long long tiles = (long long)((M + 15) / 16) * ((N + 15) / 16);
-  const int slices = (K + 31) / 32;
-  long long want = (2048 + tiles - 1) / tiles;
-  if (want > slices) want = slices;
+  const long long tiles = (long long)((M + GT - 1) / GT) * ((N + GT - 1) / GT);
+  const int slices = (K + GK - 1) / GK;
+  long long want = tiles < CU_COUNT ? (CU_COUNT + tiles - 1) / tiles : 1;
+  if (want > slices / 8) want = slices / 8;
   if (want < 1) want = 1;
   const int per = (int)((slices + want - 1) / want);
-  *kchunk = per * 32;
+  *kchunk = per * GK;
   *splits = (slices + per - 1) / per;
 }
 
 size_t mlp_gemm_work(int M, int N, int K) {
   int splits, kchunk;
   split_plan(M, N, K, &splits, &kchunk);
-  return (size_t)splits * M * N;
+  return splits > 1 ? (size_t)splits * M * N : 0;
 }
 
+size_t mlp_loss_parts(int M, int N) { return (size_t)((M + GT - 1) / GT) * ((N + GT - 1) / GT); }
+
 hipError_t mlp_gemm(const float* A, long long sam, long long sak, const float* B, long long sbk, long long sbn,
-                    float* C, int M, int N, int K, const float* bias, int act, float* work, size_t work_floats,
+                    float* C, int M, int N, int K, const GemmEpilogue& e, float* work, size_t work_floats,
                     hipStream_t s, bool split) {
   if (M < 1 || N < 1 || K < 1) return hipErrorInvalidValue;
   int splits, kchunk;
   split_plan(M, N, K, &splits, &kchunk);
-  if ((size_t)splits * M * N > work_floats) return hipErrorInvalidValue;
-  dim3 grid((unsigned)((N + 15) / 16), (unsigned)((M + 15) / 16), (unsigned)splits);
+  if (e.T || e.colsum) {
+    // the loss and the column sums need the whole of K in one workgroup
+    splits = 1;
+    kchunk = K;
+  }
+  if (splits > 1 && (size_t)splits * M * N > work_floats) return hipErrorInvalidValue;
+  GemmArgs g{A, sam, sak, B, sbk, sbn, splits > 1 ? work : C, M, N, K, kchunk, splits > 1 ? G_PART : e.T ? G_MSE : G_OUT,
+             e};
+  const long long tm = (M + GT - 1) / GT, tn = (N + GT - 1) / GT;
+  if (tm > 65535) return hipErrorInvalidValue;
+  const dim3 grid((unsigned)tn, (unsigned)tm, (unsigned)splits);
   if (split)
-    hipLaunchKernelGGL(k_gemm_bf16<true>, grid, dim3(64), 0, s, A, sam, sak, B, sbk, sbn, work, M, N, K, kchunk);
+    hipLaunchKernelGGL(k_gemm_bf16<true>, grid, dim3(256), 0, s, g);
   else
-    hipLaunchKernelGGL(k_gemm_bf16<false>, grid, dim3(64), 0, s, A, sam, sak, B, sbk, sbn, work, M, N, K, kchunk);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_gemm_sum, dim3(ew_grid((long long)M * N)), dim3(256), 0, s, work, splits, M, N, bias, act, C);
+    hipLaunchKernelGGL(k_gemm_bf16<false>, grid, dim3(256), 0, s, g);
+  hipError_t err = hipGetLastError();
+  if (err != hipSuccess || splits == 1) return err;
+  hipLaunchKernelGGL(k_gemm_sum, dim3(ew_grid((long long)M * N)), dim3(256), 0, s, work, splits, M, N, e, C);
   return hipGetLastError();
 }
 
-hipError_t mlp_tanh_back(const float* dX, const float* X, float* dZ, long long n, hipStream_t s) {
-  hipLaunchKernelGGL(k_tanh_back, dim3(ew_grid(n)), dim3(256), 0, s, dX, X, dZ, n);
-  return hipGetLastError();
-}
-
-hipError_t mlp_colsum(const float* dZ, int M, int N, float* db, hipStream_t s) {
-  hipLaunchKernelGGL(k_colsum, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, s, dZ, M, N, db);
-  return hipGetLastError();
-}
-
-hipError_t mlp_mse(const float* Y, const float* T, long long n, float* dY, float* part, int nblocks, hipStream_t s) {
-  hipLaunchKernelGGL(k_mse, dim3((unsigned)nblocks), dim3(256), 0, s, Y, T, n, dY, part);
+hipError_t mlp_loss(const float* part, int nb, double n, float* loss, int slot, int* bad, hipStream_t s) {
+  hipLaunchKernelGGL(k_loss, dim3(1), dim3(256), 0, s, part, nb, n, loss, slot, bad);
   return hipGetLastError();
 }
 
 hipError_t mlp_adam(float* p, const float* g, float* m, float* v, long long n, float lr, float b1, float b2,
-                    float eps, float c1, float c2, hipStream_t s) {
-  hipLaunchKernelGGL(k_adam, dim3(ew_grid(n)), dim3(256), 0, s, p, g, m, v, n, lr, b1, b2, eps, c1, c2);
+                    float eps, float c1, float c2, const int* bad, hipStream_t s) {
+  hipLaunchKernelGGL(k_adam, dim3(ew_grid(n)), dim3(256), 0, s, p, g, m, v, n, lr, b1, b2, eps, c1, c2, bad);
   return hipGetLastError();
 }
 
