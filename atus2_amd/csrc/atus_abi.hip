@@ -302,6 +302,29 @@ int pass_slab(atus_ctx* c, int a, int dir, int s0, int S, hipStream_t st) {
   return ATUS_OK;
 }
 
+VGeo v_geo(const atus_ctx* c) {
+  VGeo geo{};
+  geo.dim = c->dim;
+  for (int a = 0; a < 3; ++a) {
+    geo.n[a] = c->n[a];
+    geo.dx[a] = c->dx[a];
+  }
+  return geo;
+}
+
+// whether the V pass of a run of two components takes k_vcomp rather than
+// k_vfuse (block edges aside): states of up to one default slab, where it is
+// 4-19% of the step faster; larger ones run between the other passes of a
+// slab chain, where it is not (256^3: 745 us per step with either).  The rule
+// does not look at the schedule set: the two round differently, the slabs of
+// a grid must not.
+// Batches of two components follow the same rule (1024^2, 5 runs, 160 MiB:
+// the scan's step 3% slower with k_vcomp).
+bool vcomp_pair(const atus_ctx* c, int vk) {
+  return c->nc_run == 2 && 16.0 * (double)c->npts * c->ncomp <= atus_ctx::SLAB_BYTES &&
+         vcomp_ok(c->n[c->dim - 1], vk, 2);
+}
+
 // the fused inverse-z / V / forward-z pass over the x-planes [s0, s0 + S):
 // the kernel's x index counts from the slab, so n0 is shifted to keep
 // x0 = (i0 - n0/2) dx0 (n0 even), and the potential pointer moves along
@@ -313,6 +336,13 @@ int vfuse_slab(atus_ctx* c, int vk, const VArgs& va, int s0, int S, hipStream_t 
   VArgs vs = va;
   if (vs.pot) vs.pot += (long long)s0 * plane;
   ProfScope ps(c, ATUS_KFAM_VFUSE, (double)S / c->n[0], st);
+  if (!edge && vcomp_pair(c, vk)) {
+    VGeo geo = v_geo(c);
+    geo.n[0] -= 2 * s0;
+    HIP_TRY(launch_vcomp(NL, vk, 2, false, c->psi + (long long)s0 * plane, c->npts, (long long)S * c->n[1], c->tw[NL],
+                         vs, geo, lim(c, ATUS_KFAM_VFUSE), st));
+    return ATUS_OK;
+  }
   HIP_TRY(launch_vfuse(NL, vals(c, ATUS_KFAM_VFUSE), vk, c->ncomp, c->psi + (long long)s0 * plane, c->npts,
                        (long long)S * c->n[1], c->tw[NL], vs, c->n[1], c->n[0] - 2 * s0, c->dx[0], lim(c, ATUS_KFAM_VFUSE),
                        st, edge ? axis_tabs(c, 2).e0 : nullptr, edge));
@@ -1340,12 +1370,6 @@ bool vcomp_block_ok(const atus_ctx* c, int vk) {
 // separate V and kinetic steps
 int vcomp_block(atus_ctx* c, int vk, const VArgs& base, int Nk, double dt, double* t, const StepFeed& fd) {
   const int last = c->dim - 1, NL = c->n[last], N0 = c->n[0];
-  VGeo geo{};
-  geo.dim = c->dim;
-  for (int a = 0; a < 3; ++a) {
-    geo.n[a] = c->n[a];
-    geo.dx[a] = c->dx[a];
-  }
   VArgs none{};
   auto kin = [&](int f) -> int {
     ProfScope ps(c, ATUS_KFAM_KIN);
@@ -1363,7 +1387,7 @@ int vcomp_block(atus_ctx* c, int vk, const VArgs& base, int Nk, double dt, doubl
     for (int a = 1; a < last; ++a) ATUS_TRY(pass(c, a, +1, c->psi, c->psi, c->ncomp, 1.0));
     {
       ProfScope ps(c, ATUS_KFAM_VFUSE);
-      HIP_TRY(launch_vcomp(NL, vk, c->ncomp, c->psi, c->npts, c->npts / NL, c->tw[NL], va, geo,
+      HIP_TRY(launch_vcomp(NL, vk, c->ncomp, false, c->psi, c->npts, c->npts / NL, c->tw[NL], va, v_geo(c),
                            lim(c, ATUS_KFAM_VFUSE), c->stream));
     }
     for (int a = last - 1; a >= 1; --a) ATUS_TRY(pass(c, a, -1, c->psi, c->psi, c->ncomp, 1.0));
@@ -1425,9 +1449,13 @@ int single_block(atus_ctx* c, int vk, const VArgs& base, int Nk, double dt, doub
       const int edge = (m == 1 ? 1 : 0) | (m == Nk ? 2 : 0);
       {
         ProfScope ps(c, ATUS_KFAM_VFUSE);
-        HIP_TRY(launch_vfuse(NL, vals(c, ATUS_KFAM_VFUSE), vk, c->ncomp, c->psi, c->npts, c->npts / NL, c->tw[NL], va, 1,
-                             c->n[0], c->dx[0], lim(c, ATUS_KFAM_VFUSE), c->stream, edge ? axis_tabs(c, 1).e0 : nullptr,
-                             edge));
+        if (!edge && vcomp_pair(c, vk))
+          HIP_TRY(launch_vcomp(NL, vk, 2, false, c->psi, c->npts, c->npts / NL, c->tw[NL], va, v_geo(c),
+                               lim(c, ATUS_KFAM_VFUSE), c->stream));
+        else
+          HIP_TRY(launch_vfuse(NL, vals(c, ATUS_KFAM_VFUSE), vk, c->ncomp, c->psi, c->npts, c->npts / NL, c->tw[NL], va,
+                               1, c->n[0], c->dx[0], lim(c, ATUS_KFAM_VFUSE), c->stream,
+                               edge ? axis_tabs(c, 1).e0 : nullptr, edge));
       }
       ATUS_TRY(kin2d(m < Nk ? kin_tabs(c, 1) : axis_tabs(c, 0), va));
     }
@@ -1493,10 +1521,14 @@ int batch_block(atus_ctx* c, int vk, const VArgs& base, int Nk, double dt, doubl
       }
       {
         ProfScope ps(c, ATUS_KFAM_VFUSE);
-        HIP_TRY(launch_vstep_batch(NL, vals(c, ATUS_KFAM_VFUSE), false, vk, c->psi, c->npts,
-                                   (long long)B * base.pencils_per_run, c->tw[NL], kin_tabs(c, f), va, ppx, c->n[0],
-                                   c->dx[0], lim(c, ATUS_KFAM_VFUSE), c->stream,
-                                   edge ? axis_tabs(c, c->dim - 1).e0 : nullptr, edge));
+        if (!edge && vcomp_pair(c, vk))
+          HIP_TRY(launch_vcomp(NL, vk, 2, true, c->psi, c->npts, (long long)B * base.pencils_per_run, c->tw[NL], va,
+                               v_geo(c), lim(c, ATUS_KFAM_VFUSE), c->stream));
+        else
+          HIP_TRY(launch_vstep_batch(NL, vals(c, ATUS_KFAM_VFUSE), false, vk, c->psi, c->npts,
+                                     (long long)B * base.pencils_per_run, c->tw[NL], kin_tabs(c, f), va, ppx, c->n[0],
+                                     c->dx[0], lim(c, ATUS_KFAM_VFUSE), c->stream,
+                                     edge ? axis_tabs(c, c->dim - 1).e0 : nullptr, edge));
       }
       if (c->dim == 3) {
         if (last) ATUS_TRY(kin_y_slab(c, va, 0, c->n[0], c->stream));

@@ -131,6 +131,7 @@ struct atus_ctx {
   // whole grid each; -1: chosen from the size of the device's last-level
   // cache)
   int slab = -1;
+  static constexpr double SLAB_BYTES = 83886080.0;  // state of a default slab
   int slab_planes() const {
     if (dim != 3 || fs) return 0;
     int s = slab;
@@ -138,7 +139,7 @@ struct atus_ctx {
       // two slabs in flight hold about 160 MiB of the 256 MiB Infinity
       // Cache of MI355X (measured best at 256^3: 32 to 40 planes)
       const double plane = 16.0 * ncomp * n[1] * n[2];
-      s = (int)std::max(1.0, std::floor(83886080.0 / plane));
+      s = (int)std::max(1.0, std::floor(SLAB_BYTES / plane));
     }
     return s < n[0] ? s : 0;
   }

@@ -28,7 +28,7 @@ static PassCfg comp_cfg(int N, int rm, int nc, long long pencils, const Limits& 
 
 constexpr int VCOMP_MOST = 512;  // threads per workgroup
 
-template <int N, int VK, int NC>
+template <int N, int VK, int NC, bool BATCH>
 static hipError_t vcomp_go(double2* psi, long long cs, long long outer, const double2* tw, const VArgs& va,
                            const VGeo& geo, const Limits& lim, hipStream_t s) {
   constexpr int RM = comp_rm(N, NC, VCOMP_MOST);
@@ -39,9 +39,9 @@ static hipError_t vcomp_go(double2* psi, long long cs, long long outer, const do
     PassCfg c = comp_cfg(N, RM, NC, outer, lim, LB, tables_in_lds<N>());
     if (c.block.x == 0 || c.grid.x == 0) return hipErrorInvalidConfiguration;
     static bool ok = false;
-    hipError_t e = allow_lds(k_vcomp<N, RM, VK, NC, LB>, c.lds, ok);
+    hipError_t e = allow_lds(k_vcomp<N, RM, VK, NC, BATCH, LB>, c.lds, ok);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((k_vcomp<N, RM, VK, NC, LB>), c.grid, c.block, c.lds, s, psi, cs, c.g, tw, va, geo);
+    hipLaunchKernelGGL((k_vcomp<N, RM, VK, NC, BATCH, LB>), c.grid, c.block, c.lds, s, psi, cs, c.g, tw, va, geo);
     return hipGetLastError();
   }
 }
@@ -59,14 +59,16 @@ bool vcomp_ok(int N, int vk, int nc) {
   return false;
 }
 
-hipError_t launch_vcomp(int N, int vk, int nc, double2* psi, long long comp_stride, long long outer,
+hipError_t launch_vcomp(int N, int vk, int nc, bool batch, double2* psi, long long comp_stride, long long outer,
                         const double2* tw, const VArgs& va, const VGeo& geo, const Limits& lim, hipStream_t s) {
 #define ATUS_K(V, C) \
-  if (vk == V && nc == C) return vcomp_go<ATUS_N, V, C>(psi, comp_stride, outer, tw, va, geo, lim, s);
+  if (!batch && vk == V && nc == C) return vcomp_go<ATUS_N, V, C, false>(psi, comp_stride, outer, tw, va, geo, lim, s);
   switch (N) {
 #define ATUS_CASE(n)               \
   case n: {                        \
     constexpr int ATUS_N = n;      \
+    if (batch && nc == 2 && vk == V_BRAGG) return vcomp_go<n, V_BRAGG, 2, true>(psi, comp_stride, outer, tw, va, geo, lim, s); \
+    if (batch && nc == 2 && vk == V_NL_IF) return vcomp_go<n, V_NL_IF, 2, true>(psi, comp_stride, outer, tw, va, geo, lim, s); \
     ATUS_COMP_KINDS(ATUS_K) break; \
   }
     ATUS_CASE(2) ATUS_CASE(4) ATUS_CASE(8) ATUS_CASE(16) ATUS_CASE(32) ATUS_CASE(64) ATUS_CASE(128)

@@ -128,6 +128,15 @@ __device__ __forceinline__ void sincos_fast(double x, double* s, double* c) {
   }
 }
 
+// any argument by the library's routine, out of line: the callers' points
+// are unrolled, and a copy of its reduction of large arguments for each cost
+// 2-4% of the kernels that use sincos_mid
+__device__ __attribute__((noinline)) double2 sincos_large(double x) {
+  double s, c;
+  sincos(x, &s, &c);
+  return make_double2(s, c);
+}
+
 // The same where larger phases are common (kernels whose V step bounds them:
 // the 1D resident blocks, whose potential reaches far from the origin, and
 // the coupled steps of multi.hpp): for |x| < 10^6 a Cody-Waite reduction by n
@@ -177,7 +186,9 @@ __device__ __forceinline__ void sincos_mid(double x, double* s, double* c) {
     *s = (k & 2) ? -a : a;
     *c = ((k + 1) & 2) ? -b : b;
   } else {
-    sincos(x, s, c);
+    const double2 v = sincos_large(x);
+    *s = v.x;
+    *c = v.y;
   }
 }
 
@@ -425,10 +436,9 @@ __device__ __forceinline__ void bragg_point(double2& a, double2& b, double bx, d
 // the 2x2 exponential of one species of bragg_ds (bragg_ds.cpp:174-206):
 // std::complex arithmetic of the reference written out; gamma divides by
 // |d^2 + Omega^2| as the reference does
-__device__ __forceinline__ void ds_pair(double2& a, double2& b, double V11, double V22, double Om, double theta,
+__device__ __forceinline__ void ds_pair(double2& a, double2& b, double V11, double V22, double Om, double2 e,
                                         double dt) {
-  double ei, er;
-  sincos_mid(theta, &ei, &er);
+  const double er = e.x, ei = e.y;
   const double tmp1 = sqrt((V11 - V22) * (V11 - V22) + 4.0 * Om * Om);
   const double Ep = 0.5 * (V11 + V22 + tmp1);
   const double Em = 0.5 * (V11 + V22 - tmp1);
@@ -462,10 +472,28 @@ __device__ __forceinline__ void ds_diag(double2& a, double phi, double dt) {
   a.y = tmp1 * im1 + a.y * re1;
 }
 
+// What a coupled step takes from the first coordinate and the time alone:
+// the passes along another axis form it once per pencil.
+// bragg_ds: both lasers' Rabi frequencies and phase factors
+struct DsField {
+  double Om, Om2;
+  double2 e1, e2;
+};
+
+__device__ __forceinline__ DsField ds_field(double x0, const VArgs& p) {
+  DsField f;
+  const double t1 = p.t1p ? *p.t1p : p.t1;
+  f.Om = p.mode1 * p.amp0 * cos_of<true>(p.laser_k * x0 - (p.laser_domh + p.chirp_rate0 * t1) * t1 + p.phase0 / 2);
+  f.Om2 = p.mode2 * p.amp2 * cos_of<true>(p.laser_k2 * x0 - (p.laser_domh2 + p.chirp_rate2 * t1) * t1 + p.phase2 / 2);
+  sincos_mid(-0.5 * (p.laser_dk * x0 + p.phase0), &f.e1.y, &f.e1.x);
+  sincos_mid(-0.5 * (p.laser_dk2 * x0 + p.phase2), &f.e2.y, &f.e2.x);
+  return f;
+}
+
 // Bragg_single::Do_Bragg_ad of bragg_ds (bragg_ds.cpp:112-300): two species
 // of two components, couplings through all four densities, one laser per
 // species switched off by its gate
-__device__ __forceinline__ void bragg_ds_point(double2 (&a)[4], double x0, const VArgs& p) {
+__device__ __forceinline__ void bragg_ds_point(double2 (&a)[4], double x0, const DsField& f, const VArgs& p) {
   double n[4], phi[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) n[j] = a[j].x * a[j].x + a[j].y * a[j].y;
@@ -477,25 +505,17 @@ __device__ __forceinline__ void bragg_ds_point(double2 (&a)[4], double x0, const
     ph += (i < 2 ? p.beta0 : p.beta2) * x0 - p.deltaL[i];
     phi[i] = ph;
   }
-  const double t1 = p.t1p ? *p.t1p : p.t1;
-  const double Om = p.mode1 * p.amp0 * cos_of<true>(p.laser_k * x0 - (p.laser_domh + p.chirp_rate0 * t1) * t1 + p.phase0 / 2);
-  const double Om2 = p.mode2 * p.amp2 * cos_of<true>(p.laser_k2 * x0 - (p.laser_domh2 + p.chirp_rate2 * t1) * t1 + p.phase2 / 2);
-  const double th1 = -0.5 * (p.laser_dk * x0 + p.phase0);
-  const double th2 = -0.5 * (p.laser_dk2 * x0 + p.phase2);
-  if (Om == 0.0 && Om2 == 0.0) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) ds_diag(a[i], phi[i], p.dt);
-  } else if (Om == 0.0) {
+  if (f.Om == 0.0) {
     ds_diag(a[0], phi[0], p.dt);
     ds_diag(a[1], phi[1], p.dt);
-    ds_pair(a[2], a[3], phi[2], phi[3], Om2, th2, p.dt);
-  } else if (Om2 == 0.0) {
+  } else {
+    ds_pair(a[0], a[1], phi[0], phi[1], f.Om, f.e1, p.dt);
+  }
+  if (f.Om2 == 0.0) {
     ds_diag(a[2], phi[2], p.dt);
     ds_diag(a[3], phi[3], p.dt);
-    ds_pair(a[0], a[1], phi[0], phi[1], Om, th1, p.dt);
   } else {
-    ds_pair(a[0], a[1], phi[0], phi[1], Om, th1, p.dt);
-    ds_pair(a[2], a[3], phi[2], phi[3], Om2, th2, p.dt);
+    ds_pair(a[2], a[3], phi[2], phi[3], f.Om2, f.e2, p.dt);
   }
 }
 
@@ -523,9 +543,6 @@ __device__ __forceinline__ void v_point(double2 (&a)[NC], double x0, long long l
 #pragma unroll
     for (int c = 0; c < NC; ++c) extra[c] = (c < NC / 2 ? p.beta0 : p.beta2) * x0 - p.deltaL[c];
     nl_point<NC, false, MID>(a, extra, p);
-  } else if constexpr (VK == V_BRAGG_DS) {
-    static_assert(NC == 4, "the two-species Bragg step has four components");
-    bragg_ds_point(a, x0, p);
   }
 }
 
@@ -641,11 +658,14 @@ __device__ __forceinline__ void three_state_diag(double2 (&H)[NC][NC], const dou
 // CRT_Base_IF::Numerical_Bragg (CRT_Base_IF.h:426-527): state 0 coupled to
 // state i+1 by the lasers of wave number +-laser_k and chirp +-chirp_rate,
 // at t = Get_t() before the step
+struct NumField {
+  double2 e[2];  // element (i + 1, 0)
+};
+
 template <int NC>
-__device__ __forceinline__ void num_bragg_point(double2 (&a)[NC], double x0, double bx, const VArgs& p) {
+__device__ __forceinline__ NumField num_bragg_field(double x0, const VArgs& p) {
   static_assert(NC == 2 || NC == 3, "the numerical Bragg step has two or three states");
-  double2 H[NC][NC];
-  three_state_diag<NC>(H, a, bx, p);
+  NumField f;
   const double t = p.t0;
 #pragma unroll
   for (int i = 0; i < NC - 1; ++i) {
@@ -653,46 +673,71 @@ __device__ __forceinline__ void num_bragg_point(double2 (&a)[NC], double x0, dou
     const double cr = i == 0 ? p.chirp_rate0 : -p.chirp_rate0;
     double sn, cs;
     sincos_mid((-p.laser_domh + cr * t) * t + k * x0 - 0.5 * p.phase0, &sn, &cs);
-    const double er = p.amp0 * cs / 2 + p.amp1 * cs / 2;
-    const double ei = p.amp0 * sn / 2 - p.amp1 * sn / 2;
-    H[i + 1][0] = make_double2(er, ei);
-    H[0][i + 1] = make_double2(er, -ei);
+    f.e[i] = make_double2(p.amp0 * cs / 2 + p.amp1 * cs / 2, p.amp0 * sn / 2 - p.amp1 * sn / 2);
+  }
+  return f;
+}
+
+template <int NC>
+__device__ __forceinline__ void num_bragg_point(double2 (&a)[NC], double bx, const NumField& f, const VArgs& p) {
+  double2 H[NC][NC];
+  three_state_diag<NC>(H, a, bx, p);
+#pragma unroll
+  for (int i = 0; i < NC - 1; ++i) {
+    H[i + 1][0] = f.e[i];
+    H[0][i + 1] = make_double2(f.e[i].x, -f.e[i].y);
   }
   herm_expm_apply<NC>(H, p.dt, a);
 }
 
 // CRT_Base_IF::Numerical_Raman (CRT_Base_IF.h:534-632): states 0 and 1
 // coupled to state 2, which carries the detuning laser_domh
+__device__ __forceinline__ double2 raman_field(double x0, const VArgs& p) {
+  double2 e;
+  sincos_mid(p.laser_k * x0, &e.y, &e.x);
+  return e;
+}
+
 template <int NC>
-__device__ __forceinline__ void raman_point(double2 (&a)[NC], double x0, double bx, const VArgs& p) {
+__device__ __forceinline__ void raman_point(double2 (&a)[NC], double bx, double2 e, const VArgs& p) {
   static_assert(NC >= 3, "the Raman step couples three states");
   double2 H[NC][NC];
   three_state_diag<NC>(H, a, bx, p);
   H[2][2].x = H[2][2].x + p.laser_domh;
-  double sn, cs;
-  sincos_mid(p.laser_k * x0, &sn, &cs);
-  H[0][2] = make_double2(p.amp0 / 2 * cs, p.amp0 / 2 * sn);
-  H[2][0] = make_double2(p.amp0 / 2 * cs, -(p.amp0 / 2 * sn));
-  H[1][2] = make_double2(p.amp1 / 2 * cs, -(p.amp1 / 2 * sn));
-  H[2][1] = make_double2(p.amp1 / 2 * cs, p.amp1 / 2 * sn);
+  H[0][2] = make_double2(p.amp0 / 2 * e.x, p.amp0 / 2 * e.y);
+  H[2][0] = make_double2(p.amp0 / 2 * e.x, -(p.amp0 / 2 * e.y));
+  H[1][2] = make_double2(p.amp1 / 2 * e.x, -(p.amp1 / 2 * e.y));
+  H[2][1] = make_double2(p.amp1 / 2 * e.x, p.amp1 / 2 * e.y);
   herm_expm_apply<NC>(H, p.dt, a);
 }
 
 // Bragg_double::Do_Double_Bragg_ad (double_bragg.cpp:108-249): the
 // reference's closed-form 3x3 exponential, its operations in its order
 // (O23 and O32 take their phases as written there)
-__device__ __forceinline__ void dbragg_point(double2 (&a)[3], double x0, double bx, const VArgs& p) {
-  const double dt = p.dt, t1 = p.t1;
+struct DbField {
+  double Op, Om;
+  double e0, e1;
+};
+
+__device__ __forceinline__ DbField dbragg_field(double x0, const VArgs& p) {
+  DbField f;
+  const double t1 = p.t1;
   const double F = p.F < 0.0 ? 0.0 : p.F;
+  double dw = p.laser_domh + p.chirp_rate0 * t1;
+  f.Op = F * p.amp0 * cos_of<true>(p.laser_k * x0 - dw * t1 - p.phase0 / 2);
+  dw = p.laser_domh - p.chirp_rate0 * t1;
+  f.Om = F * p.amp0 * cos_of<true>(-p.laser_k * x0 - dw * t1 - p.phase0 / 2);
+  sincos_mid(-0.5 * p.laser_dk * x0, &f.e1, &f.e0);
+  return f;
+}
+
+__device__ __forceinline__ void dbragg_point(double2 (&a)[3], double bx, const DbField& f, const VArgs& p) {
+  const double dt = p.dt, Op = f.Op, Om = f.Om;
   const double n1 = a[0].x * a[0].x + a[0].y * a[0].y;
   const double n2 = a[1].x * a[1].x + a[1].y * a[1].y;
   const double n3 = a[2].x * a[2].x + a[2].y * a[2].y;
   const double V11 = p.gs[0] * n1 + p.gs[1] * n2 + p.gs[2] * n3 + bx;
   const double V22 = p.gs[3] * n1 + p.gs[4] * n2 + p.gs[5] * n3 - p.deltaL[1] + bx;
-  double dw = p.laser_domh + p.chirp_rate0 * t1;
-  const double Op = F * p.amp0 * cos_of<true>(p.laser_k * x0 - dw * t1 - p.phase0 / 2);
-  dw = p.laser_domh - p.chirp_rate0 * t1;
-  const double Om = F * p.amp0 * cos_of<true>(-p.laser_k * x0 - dw * t1 - p.phase0 / 2);
   double im1, re1, tmp1, tmp2;
   if (Om == 0.0 && Op == 0.0) {
     sincos_mid(-dt * V11, &im1, &re1);
@@ -708,8 +753,7 @@ __device__ __forceinline__ void dbragg_point(double2 (&a)[3], double x0, double 
     }
     return;
   }
-  sincos_mid(-0.5 * p.laser_dk * x0, &im1, &re1);
-  const double e0 = re1, e1 = im1;
+  const double e0 = f.e0, e1 = f.e1;
   tmp1 = sqrt((V11 - V22) * (V11 - V22) + 4.0 * (Op * Op + Om * Om));
   const double E1 = 0.5 * (V11 + V22 + tmp1);
   const double E2 = 0.5 * (V11 + V22 - tmp1);
@@ -763,6 +807,53 @@ __device__ __forceinline__ void dbragg_point(double2 (&a)[3], double x0, double 
   a[1].y = (O21r * q1.y + O21i * q1.x) + (O22r * q2.y + O22i * q2.x) + (O23r * q3.y + O23i * q3.x);
   a[2].x = (O31r * q1.x - O31i * q1.y) + (O32r * q2.x - O32i * q2.y) + (O33r * q3.x - O33i * q3.y);
   a[2].y = (O31r * q1.y + O31i * q1.x) + (O32r * q2.y + O32i * q2.x) + (O33r * q3.y + O33i * q3.x);
+}
+
+// what any V step takes from the first coordinate alone, and the step on one
+// point: bx = beta.x of the three-state steps, l the point's linear index.
+// MID (the uncoupled and the Bragg step): sincos_mid.
+struct NoField {};
+struct BraggField {
+  double Om;
+  double2 eta;
+};
+
+template <int VK, int NC, bool MID>
+__device__ __forceinline__ auto v_field(double x0, const VArgs& va) {
+  if constexpr (VK == V_BRAGG) {
+    BraggField f;
+    bragg_field<MID>(x0, va, f.Om, f.eta);
+    return f;
+  } else if constexpr (VK == V_BRAGG_DS) {
+    return ds_field(x0, va);
+  } else if constexpr (VK == V_DBRAGG) {
+    return dbragg_field(x0, va);
+  } else if constexpr (VK == V_NUM_BRAGG) {
+    return num_bragg_field<NC>(x0, va);
+  } else if constexpr (VK == V_RAMAN) {
+    return raman_field(x0, va);
+  } else {
+    return NoField{};
+  }
+}
+
+template <int VK, int NC, bool MID, class Field>
+__device__ __forceinline__ void any_point(double2 (&a)[NC], double x0, double bx, long long l, const Field& f,
+                                          const VArgs& va) {
+  if constexpr (VK == V_BRAGG) {
+    v_point<VK, NC, MID>(a, x0, l, va, f.Om, f.eta);
+  } else if constexpr (VK == V_BRAGG_DS) {
+    static_assert(NC == 4, "the two-species Bragg step has four components");
+    bragg_ds_point(a, x0, f, va);
+  } else if constexpr (VK == V_DBRAGG) {
+    dbragg_point(a, bx, f, va);
+  } else if constexpr (VK == V_NUM_BRAGG) {
+    num_bragg_point<NC>(a, bx, f, va);
+  } else if constexpr (VK == V_RAMAN) {
+    raman_point<NC>(a, bx, f, va);
+  } else {
+    v_point<VK, NC, MID>(a, x0, l, va, 0.0, make_double2(1.0, 0.0));
+  }
 }
 
 // ------------------------------------------------------------ k_pass
@@ -1204,18 +1295,9 @@ __global__ __launch_bounds__(256) void k_point(double2* __restrict__ psi, Grid g
 #pragma unroll
     for (int c = 0; c < NC; ++c) a[c] = psi[c * gr.npts + l];
     const double x0 = x0_of(l, gr);
-    double Om = 0.0;
-    double2 eta = make_double2(1.0, 0.0);
-    if constexpr (VK == V_BRAGG) bragg_field(x0, va, Om, eta);
-    if constexpr (VK == V_DBRAGG) {
-      dbragg_point(a, x0, beta_dot_x(l, gr, va.beta), va);
-    } else if constexpr (VK == V_NUM_BRAGG) {
-      num_bragg_point<NC>(a, x0, beta_dot_x(l, gr, va.beta), va);
-    } else if constexpr (VK == V_RAMAN) {
-      raman_point<NC>(a, x0, beta_dot_x(l, gr, va.beta), va);
-    } else {
-      v_point<VK, NC>(a, x0, l, va, Om, eta);
-    }
+    double bx = 0.0;
+    if constexpr (VK == V_DBRAGG || VK == V_NUM_BRAGG || VK == V_RAMAN) bx = beta_dot_x(l, gr, va.beta);
+    any_point<VK, NC, false>(a, x0, bx, l, v_field<VK, NC, false>(x0, va), va);
 #pragma unroll
     for (int c = 0; c < NC; ++c) psi[c * gr.npts + l] = a[c];
   }

@@ -49,7 +49,12 @@ constexpr int CU_COUNT = 256;  // compute units of MI355X
 // what a launch may use: LDS bytes per workgroup, and threads per
 // workgroup at most (the pencils per workgroup follow as threads / P, at
 // least one pencil).  0: as many as the kernel's launch bounds allow, halved
-// down to one wavefront while the pass has fewer than two workgroups per CU.
+// down to one wavefront while the pass has fewer than four workgroups per CU
+// (32x64x32, two components: the kinetic pass ran 32 workgroups of 256
+// threads, 7.2 us, and takes 5.0 in 256 of 64; 64^3, four components: the
+// middle axis 2.7% of the step), but not below four columns of a strided
+// pass, 64-byte segments of a row (512^2, three components: 2.5% of the step
+// faster with four than with two).
 struct Limits {
   size_t lds;
   int threads;
@@ -74,7 +79,8 @@ inline PassCfg make_pass_cfg(int N, int rm, long long inner, long long outer, in
     if (t < P) t = P < max_threads ? P : max_threads;
   } else {
     const long long pencils = inner * outer * ycount;
-    while (t > 64 && t > P && pencils * P < 2LL * CU_COUNT * t) t >>= 1;
+    const int least = inner > 1 ? 4 * P : P;
+    while (t > 64 && t > least && pencils * P < 4LL * CU_COUNT * t) t >>= 1;
   }
   return make_pass_cfg(N, rm, inner, outer, ycount, lim.lds, ntables, t, table_elems, min_threads);
 }
@@ -134,9 +140,10 @@ hipError_t launch_block1d(int vk, bool batch, double2* psi, long long cs, long l
 // the same passes with the components on thread groups of their own
 // (multi.hpp); *_ok: whether the kind, component count and length are
 // covered.  launch_vcomp: inverse / V / forward along the last axis of a
-// 2D/3D grid, `outer` pencils; launch_bcomp: blocks of 1D runs
+// 2D/3D grid, `outer` pencils (of all runs of a batch); launch_bcomp: blocks
+// of 1D runs
 bool vcomp_ok(int N, int vk, int nc);
-hipError_t launch_vcomp(int N, int vk, int nc, double2* psi, long long comp_stride, long long outer,
+hipError_t launch_vcomp(int N, int vk, int nc, bool batch, double2* psi, long long comp_stride, long long outer,
                         const double2* tw, const VArgs& va, const VGeo& geo, const Limits& lim, hipStream_t s);
 bool bcomp_ok(int N, int vk, int nc);
 hipError_t launch_bcomp(int N, int vk, int nc, bool batch, double2* psi, long long comp_stride, long long runs,

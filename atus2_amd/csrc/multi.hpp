@@ -17,23 +17,6 @@ __host__ __device__ constexpr int comp_rm(int N, int NC, int most) {
   return (N >= 32 && NC * (N / 16) <= most) ? 16 : 0;
 }
 
-// V step of any kind on one point; bx = beta.x of the three-state steps
-template <int VK, int NC>
-__device__ __forceinline__ void any_point(double2 (&a)[NC], double x0, double bx, long long l, const VArgs& va) {
-  if constexpr (VK == V_DBRAGG) {
-    dbragg_point(a, x0, bx, va);
-  } else if constexpr (VK == V_NUM_BRAGG) {
-    num_bragg_point<NC>(a, x0, bx, va);
-  } else if constexpr (VK == V_RAMAN) {
-    raman_point<NC>(a, x0, bx, va);
-  } else {
-    double Om = 0.0;
-    double2 eta = make_double2(1.0, 0.0);
-    if constexpr (VK == V_BRAGG) bragg_field<true>(x0, va, Om, eta);
-    v_point<VK, NC, true>(a, x0, l, va, Om, eta);
-  }
-}
-
 __device__ __forceinline__ double2 sel(bool b, double2 x, double2 y) {
   return make_double2(b ? x.x : y.x, b ? x.y : y.y);
 }
@@ -101,8 +84,14 @@ __device__ __forceinline__ void comp_vstep(double2 (&v)[(Plan<N, RM>::R)], int c
 }
 
 // inverse DFT along the last axis of a 2D/3D grid, V step, forward DFT.
-// Workgroup: g.T pencils of NC x P threads.
-template <int N, int RM, int VK, int NC, int LB>
+// Workgroup: g.T pencils of NC x P threads.  BATCH: the pencils of all runs
+// of a batch, each with its run's parameters.  Against k_vfuse, which holds
+// both components of a pencil in the same threads (144 registers, three
+// waves per SIMD; here 112, four), a Bragg step takes 12.7 us for 15.6 at
+// 128^2, 23.6 for 27.3 at 512^2, 28.6 for 31.2 at 64^3, 103.9 for 108.5 at
+// 128^3; between the other stream's passes of a slab chain (256^3) the two
+// are equal.
+template <int N, int RM, int VK, int NC, bool BATCH, int LB>
 __global__ __launch_bounds__(LB) void k_vcomp(double2* __restrict__ psi, long long comp_stride, AxisGeo g,
                                               const double2* __restrict__ tw, VArgs va, VGeo geo) {
   extern __shared__ double2 lds_all[];
@@ -115,11 +104,19 @@ __global__ __launch_bounds__(LB) void k_vcomp(double2* __restrict__ psi, long lo
   double2* region = lds_all + p * g.ls;
   const int cs = g.T * g.ls;
   const double2* twl = stage_table<N>(lds_all + (size_t)NC * cs, fft_tw<N, RM>(tw));
+  long long own = pid;  // pencil of its run
+  if constexpr (BATCH) {
+    const long long r = pid / va.pencils_per_run;
+    own = pid - r * va.pencils_per_run;
+    if (valid) bind_run(va, r);
+    psi += r * va.run_shift;
+  }
   double2 v[R];
   load_pencil<N, RM>(v, psi + c * comp_stride, pid * N, 1, t, valid);
   const unsigned ppx = geo.dim == 3 ? (unsigned)geo.n[1] : 1u;
-  const int i0 = (int)((unsigned)pid / ppx), i1 = (int)((unsigned)pid % ppx);
+  const int i0 = (int)((unsigned)own / ppx), i1 = (int)((unsigned)own % ppx);
   const double x0 = (double)(i0 - geo.n[0] / 2) * geo.dx[0];
+  const auto field = v_field<VK, NC, false>(x0, va);
   if constexpr (tables_in_lds<N>()) __syncthreads();
   fft_pencil<N, RM, +1, WAVE>(v, t, region + c * cs, fresh_tw<N>(twl));
   comp_vstep<N, RM, NC, WAVE>(v, c, t, region, cs, valid, [&](double2(&a)[NC], int j) {
@@ -131,7 +128,7 @@ __global__ __launch_bounds__(LB) void k_vcomp(double2* __restrict__ psi, long lo
       const int last = geo.dim - 1;
       bx += va.beta[last] * ((double)(j - N / 2) * geo.dx[last]);
     }
-    any_point<VK, NC>(a, x0, bx, pid * N + j, va);
+    any_point<VK, NC, false>(a, x0, bx, pid * N + j, field, va);
   });
   fft_pencil<N, RM, -1, WAVE>(v, t, region + c * cs, fresh_tw<N>(twl));
   store_pencil<N, RM>(v, psi + c * comp_stride, pid * N, 1, t, valid);
@@ -223,13 +220,14 @@ __global__ __launch_bounds__(LB) void k_bcomp(double2* __restrict__ psi, long lo
           const double extra[1] = {pot[i]};
           nl_point<1, true, true>(a, extra, va);
         } else {
-          any_point<VK, 1>(a, (double)(u + P * i - N / 2) * dx0, 0.0, u + P * i, va);
+          any_point<VK, 1, true>(a, (double)(u + P * i - N / 2) * dx0, 0.0, u + P * i, NoField{}, va);
         }
         v[i] = a[0];
       }
     } else {
       comp_vstep<N, RM, NC, WAVE>(v, c, u, region, cs, valid, [&](double2(&a)[NC], int j) {
-        any_point<VK, NC>(a, (double)(j - N / 2) * dx0, 0.0, j, va);
+        const double x0 = (double)(j - N / 2) * dx0;
+        any_point<VK, NC, true>(a, x0, 0.0, j, v_field<VK, NC, true>(x0, va), va);
       });
     }
     const bool last = s + 1 == st.Nk;

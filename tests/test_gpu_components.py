@@ -20,7 +20,7 @@ KINDS = [("freeprop", 2, True), ("freeprop", 3, False), ("freeprop", 4, True), (
          ("num", 2, True), ("num", 3, False), ("raman", 3, False), ("raman", 4, False)]
 
 
-@pytest.mark.parametrize("kind,nc,two", KINDS)
+@pytest.mark.parametrize("kind,nc,two", KINDS + [("freeprop", 2, False), ("if", 2, False), ("bragg", 2, False)])
 @pytest.mark.parametrize("shape", [(2, 2), (8, 4), (4, 8), (16, 16), (2, 1024), (2, 2048), (2, 4096), (64, 256),
                                    (2, 4, 8), (8, 2, 32), (4, 16, 512), (256, 512)])
 def test_2d_3d_blocks_equal_single_steps(shape, kind, nc, two):
