@@ -13,6 +13,7 @@
 #include "../../include/atus_hip.h"
 #include "ctx.hpp"
 #include "kernels_misc.hpp"
+#include "staging.hpp"
 
 using namespace atus;
 using atus_host::fail;
@@ -858,6 +859,7 @@ int ctx_create(atus_ctx** out, int dim, const long long n[3], const double dx[3]
     }
   }
   atus_ctx* c = new atus_ctx();
+  atus_host::staging().ref();
   c->dim = dim;
   c->ncomp = ncomp;
   c->nc_run = nc_run;
@@ -969,6 +971,7 @@ int atus_ctx_destroy(atus_ctx* c) {
   for (hipStream_t x : c->xstream)
     if (x) (void)hipStreamDestroy(x);
   if (c->stream) (void)hipStreamDestroy(c->stream);
+  atus_host::staging().unref();
   delete c;
   return ATUS_OK;
 }
@@ -992,7 +995,13 @@ int atus_download(atus_ctx* c, int comp, double* host) {
   ATUS_TRY(check_ctx(c));
   ATUS_TRY(check_comp(c, comp));
   if (!host) return fail(ATUS_ERR_ARG, "null host pointer");
-  HIP_TRY(hipMemcpyAsync(host, c->psi + comp * c->npts, sizeof(double2) * c->npts, hipMemcpyDeviceToHost, c->stream));
+  const double2* src = c->psi + comp * c->npts;
+  const hipError_t e = atus_host::staging().to_host(host, src, sizeof(double2) * c->npts, c->stream, c->device);
+  if (e != hipErrorNotReady) {
+    HIP_TRY(e);
+    return ATUS_OK;
+  }
+  HIP_TRY(hipMemcpyAsync(host, src, sizeof(double2) * c->npts, hipMemcpyDeviceToHost, c->stream));
   HIP_TRY(hipStreamSynchronize(c->stream));
   return ATUS_OK;
 }
