@@ -270,8 +270,9 @@ int atus_tune_threads(atus_ctx *ctx, int family, int threads);
  * The results do not change. */
 int atus_set_slab(atus_ctx *ctx, int planes);
 /* scheduling of 1D blocks (no reference counterpart): grids of up to 4096
- * points (single runs of one or two components, and batches) run a whole
- * block of atus_run_block / atus_batch_run_block / a graph in one launch,
+ * points (one or two components, and batches) and of up to 2048 points
+ * (three or four components that only the nonlinearity couples) run a whole
+ * block of atus_run_block(_ds) / atus_batch_run_block / a graph in one launch,
  * each run's pencil resident in registers from the first half kinetic step
  * to the last; the per-step t1 and amplitudes are evaluated on the host
  * with the per-step bookkeeping and uploaded before the launch.  on = 1
