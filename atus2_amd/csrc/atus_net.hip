@@ -113,6 +113,24 @@ int adam_step(atus_net* n, long long step, float lr) {
   return ATUS_OK;
 }
 
+// floats of workspace the products of any batch up to max_batch need.  A
+// product's splits depend on its tiles, and fewer rows of tiles take more
+// splits (256 x 64 x 32768: 64 of them, 192 rows 86), so the largest batch
+// need not need the most: of the batches with the same rows of tiles it is
+// the largest
+size_t net_work(const int dims[5], int max_batch) {
+  size_t work = 0;
+  for (int b = MLP_TILE;; b += MLP_TILE) {
+    const int B = std::min(b, max_batch);
+    for (int l = 0; l < 4; ++l) {
+      const int in = dims[l], o = dims[l + 1];
+      work = std::max(work, mlp_gemm_work(B, o, in));             // forward
+      if (l > 0) work = std::max(work, mlp_gemm_work(B, in, o));  // dX
+    }
+    if (B == max_batch) return work;
+  }
+}
+
 int check_batch(atus_net* n, int B) {
   if (B < 1 || B > n->max_batch)
     return fail(ATUS_ERR_ARG, "batch must be 1.." + std::to_string(n->max_batch));
@@ -148,13 +166,7 @@ int atus_net_create(atus_net** out, int n_in, int h1, int h2, int h3, int n_out,
   };
   if (hipGetDevice(&n->device) != hipSuccess) return bail(ATUS_ERR_HIP, "no HIP device");
   if (hipStreamCreateWithFlags(&n->stream, hipStreamNonBlocking) != hipSuccess) return bail(ATUS_ERR_HIP, "stream");
-  size_t work = 0;
-  for (int l = 0; l < 4; ++l) {
-    const int in = dims[l], o = dims[l + 1];
-    work = std::max(work, mlp_gemm_work(max_batch, o, in));  // forward
-    work = std::max(work, mlp_gemm_work(in, o, max_batch));  // dW
-    work = std::max(work, mlp_gemm_work(max_batch, in, o));  // dX
-  }
+  const size_t work = net_work(dims, max_batch);
   n->work_floats = work;
   n->idx_cap = std::max(65536, max_batch);
   bool ok = hipMalloc(&n->p, sizeof(float) * n->np) == hipSuccess && hipMalloc(&n->g, sizeof(float) * n->np) == hipSuccess &&

@@ -24,7 +24,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 // in flight in registers while this one is multiplied.  The large products
 // (256 x 32768 x 64 and its two transposes) stream their operands; what
 // follows them rides in their epilogues rather than in passes of its own.
-constexpr int GT = 64;        // tile edge
+constexpr int GT = MLP_TILE;  // tile edge
 constexpr int GK = 32;        // slice along k
 constexpr int GP = GK + 8;    // LDS row pitch: 16-byte rows on distinct banks
 

@@ -20,6 +20,7 @@ struct GemmEpilogue {
   float* loss = nullptr;
   float* colsum = nullptr;      // column sums of B
 };
+constexpr int MLP_TILE = 64;  // rows and columns of a product's tile
 // floats of workspace mlp_gemm needs for an M x N x K product
 size_t mlp_gemm_work(int M, int N, int K);
 // loss partials of an M x N output

@@ -41,6 +41,34 @@ def test_forward_and_gradients(dims, batch, terms):
             assert e < 8 * 2 * u * np.linalg.norm(gref[o:o + n]), (o, n, e)
 
 
+@pytest.mark.parametrize("dims,max_batch,batches", [((4, 256, 256, 64, 32768), 256, (128, 191, 192)),
+                                                    ((4, 256, 256, 64, 32768), 200, (101, 128, 192)),
+                                                    ((4, 64, 256, 256, 32768), 65, (33, 64)),
+                                                    ((4, 16, 16, 17, 4100), 300, (1, 64, 128, 193, 256))])
+def test_batches_below_the_largest(dims, max_batch, batches):
+    # fewer rows of tiles are split into more parts along k: the workspace
+    # holds those of every batch, not of the largest alone.  Tolerances as in
+    # test_forward_and_gradients.
+    from atus2_amd import hip
+    rng = np.random.default_rng(5)
+    u = 2.0 ** -17
+    with hip.Net(dims, max_batch=max_batch, seed=3) as net:
+        p = net.get_params()
+        for batch in batches:
+            x = rng.uniform(-1, 1, (batch, dims[0])).astype(np.float32)
+            t = rng.standard_normal((batch, dims[4])).astype(np.float32)
+            net.set_params(p)
+            loss, g = net.gradients(x, t)
+            lref, gref = M.loss_and_gradients(p, dims, x, t, None)
+            assert abs(loss / lref - 1) < 2 * 4 * 2 * u
+            for wo, ws, bo, bn in M.layout(dims)[0]:
+                for o, n in ((wo, ws[0] * ws[1]), (bo, bn)):
+                    e = np.linalg.norm(g[o:o + n] - gref[o:o + n])
+                    assert e < 8 * 2 * u * np.linalg.norm(gref[o:o + n]), (batch, o, n, e)
+            net.set_data(x, t)
+            assert abs(net.train(1, batch, 1e-3)[0] / lref - 1) < 2 * 4 * 2 * u
+
+
 def test_training_in_chunks_equals_single_steps():
     # 300 steps run as two chunks; the same steps one call each give the
     # same losses (constant rate, the whole set as one batch)
