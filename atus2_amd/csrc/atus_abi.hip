@@ -84,14 +84,22 @@ namespace {
 // the family's tuned threads per workgroup (atus_tune_threads)
 Limits lim(const atus_ctx* c, int fam) { return Limits{c->max_lds, c->wg[fam]}; }
 
+// values of one run's state.  What rounds differently is chosen by it, never
+// by the size of a batch: a run gives the same bits whatever runs share its
+// batch
+long long run_values(const atus_ctx* c) { return c->npts * c->nc_run; }
+
 // values per thread of kernel family fam: the tuned choice, else 8 for the
-// strided passes and the V pass (which spills at 16), and 16, half the
-// exchanges, for the contiguous passes and the kinetic step of a state large
-// enough to give every CU two workgroups of 256 threads all the same
+// strided passes and the V pass (which spills at 16), and for the contiguous
+// passes and the kinetic step 16, half the exchanges, for runs large enough
+// to give every CU two workgroups of 256 threads all the same.  The smaller
+// runs keep 8 in large batches too (us per step, 8 and 16 values: five runs
+// of 512^2 48 and 56, twenty 138 and 149, five of 2048 x 256 95 and 107, ten
+// of 64^3 118 and 124; 1024^2, five runs: 169 and 164)
 int vals(const atus_ctx* c, int fam) {
   if (c->rm[fam]) return c->rm[fam];
   if (fam == ATUS_KFAM_PASS_STRIDED || fam == ATUS_KFAM_VFUSE) return 8;
-  return c->npts * c->ncomp >= 2LL * CU_COUNT * 256 * 16 ? 16 : 8;
+  return run_values(c) >= 2LL * CU_COUNT * 256 * 16 ? 16 : 8;
 }
 
 int check_ctx(atus_ctx* c) {
@@ -314,16 +322,21 @@ VGeo v_geo(const atus_ctx* c) {
 }
 
 // whether the V pass of a run of two components takes k_vcomp rather than
-// k_vfuse (block edges aside): states of up to one default slab, where it is
+// k_vfuse (block edges aside): runs of up to one default slab, where it is
 // 4-19% of the step faster; larger ones run between the other passes of a
 // slab chain, where it is not (256^3: 745 us per step with either).  The rule
 // does not look at the schedule set: the two round differently, the slabs of
 // a grid must not.
-// Batches of two components follow the same rule (1024^2, 5 runs, 160 MiB:
-// the scan's step 3% slower with k_vcomp).
+// In batch contexts, up to 512 points along the last axis (us per step, k_vfuse
+// and k_vcomp: 128^2, 40 runs 38.5 and 36.3; 64^3, 20 runs 222 and 214; 512^2,
+// one run 27.0 and 24.8, ten 80 either way, twenty 138 and 142): beyond that
+// one or two runs alone gain (1024^2: 47.6 and 46.3, 82.1 and 76.2), the many
+// of a scan lose (512 runs, 43 of them 1024^2: 100.7 ms per 50 steps against
+// 97.2; 256 x 2048, 5 runs: 97 and 104).
 bool vcomp_pair(const atus_ctx* c, int vk) {
-  return c->nc_run == 2 && 16.0 * (double)c->npts * c->ncomp <= atus_ctx::SLAB_BYTES &&
-         vcomp_ok(c->n[c->dim - 1], vk, 2);
+  const int NL = c->n[c->dim - 1];
+  if (c->nc_run != 2 || 16.0 * (double)run_values(c) > atus_ctx::SLAB_BYTES) return false;
+  return (!c->runs || NL <= 512) && vcomp_ok(NL, vk, 2);
 }
 
 // the fused inverse-z / V / forward-z pass over the x-planes [s0, s0 + S):

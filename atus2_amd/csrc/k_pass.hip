@@ -131,7 +131,12 @@ static hipError_t rabi_nr(int axis, const double2* src, long long seg, int nseg,
   PassCfg c;
   if (axis == 2) c = make_pass_cfg(N, RM, 1, (long long)rb.n[0] * rb.n[1], nseg, lim);
   else if (axis == 1) c = make_pass_cfg(N, RM, rb.len[2], rb.n[0], nseg, lim);
-  else c = make_pass_cfg(N, RM, (long long)rb.len[1] * rb.len[2], 1, nseg, lim, 1, 256, -1, 64);
+  else {
+    // one segment's columns alone set the workgroup: its partial sums, and so
+    // the rounding of a run's populations, do not depend on the batch
+    c = make_pass_cfg(N, RM, (long long)rb.len[1] * rb.len[2], 1, 1, lim, 1, 256, -1, 64);
+    c.grid.y = (unsigned)nseg;
+  }
   if (c.block.x == 0 || c.block.x > 256 || c.grid.x == 0) return hipErrorInvalidConfiguration;
   static bool ok[3] = {false, false, false};
   hipError_t e;

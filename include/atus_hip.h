@@ -252,7 +252,8 @@ int atus_run_block_profiled(atus_ctx *ctx, const atus_step_params *sp, int Nk, d
  * family (ATUS_KFAM_*; the Sobolev minimiser's iteration takes 8 always).  16 halves
  * the LDS exchanges, 8 halves the registers per thread.  Defaults: 8 for
  * the strided passes and the fused V pass, and for the contiguous passes
- * and the kinetic step 16, or 8 below 2^21 values of state. */
+ * and the kinetic step 16, or 8 where a run's state has fewer than 2^21
+ * values. */
 int atus_tune(atus_ctx *ctx, int family, int values_per_thread);
 /* tile choice of a kernel family (no reference counterpart): at most
  * `threads` threads per workgroup (64, 128, 256 or 512; 0, the default: as
