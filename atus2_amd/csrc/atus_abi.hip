@@ -571,14 +571,15 @@ int reduce_seg(atus_ctx* c, const Fn& fn, long long n, long long seg_stride, int
 struct Marginals {
   std::vector<double> x[3], k[3];
   double phase = 0;
-  // sum of f(coordinate) times the density
+  // sum of f(coordinate) times the density, over up to 4096 terms one after
+  // another: in long double, so that the chain adds no error of its own
   static double moment(const std::vector<double>& d, const std::vector<double>& q, double mu, int power) {
-    double s = 0.0;
+    long double s = 0.0L;
     for (size_t j = 0; j < d.size(); ++j) {
-      const double e = q[j] - mu;
-      s += d[j] * (power == 0 ? 1.0 : power == 1 ? e : e * e);
+      const long double e = (long double)q[j] - mu;
+      s += d[j] * (power == 0 ? 1.0L : power == 1 ? e : e * e);
     }
-    return s;
+    return (double)s;
   }
 };
 
@@ -645,8 +646,9 @@ int marginals(atus_ctx* c, const double2* p, bool phase, Marginals& m) {
     }
     o += n;
   }
-  m.phase = 0;
-  for (size_t b = 0; b < nph; ++b) m.phase += h[2 * nout + b];
+  long double phsum = 0.0L;
+  for (size_t b = 0; b < nph; ++b) phsum += h[2 * nout + b];
+  m.phase = (double)phsum;
   return ATUS_OK;
 }
 

@@ -47,12 +47,14 @@ __global__ __launch_bounds__(256) void k_marginal(const double2* __restrict__ ps
     }
     double2 v[R];
     load_pencil<N, RM>(v, psi, base, stride, t, valid);
+    double phi = 0.0;
 #pragma unroll
     for (int i = 0; i < R; ++i) {
       const double d = v[i].x * v[i].x + v[i].y * v[i].y;
       ax[i] += d;
-      if constexpr (PHASE) ph += atan2(v[i].y, v[i].x) * d;
+      if constexpr (PHASE) phi += atan2(v[i].y, v[i].x) * d;
     }
+    if constexpr (PHASE) ph += phi;
     fft_pencil<N, RM, -1, WAVE>(v, t, lds, fresh_tw<N>(twl));
 #pragma unroll
     for (int i = 0; i < R; ++i) ak[i] += v[i].x * v[i].x + v[i].y * v[i].y;
@@ -71,11 +73,12 @@ __global__ __launch_bounds__(256) void k_marginal(const double2* __restrict__ ps
     double* sh = reinterpret_cast<double*>(lds_all);
     sh[threadIdx.x] = ph;
     __syncthreads();
-    if (threadIdx.x == 0) {
-      double s = 0.0;
-      for (int q = 0; q < (int)blockDim.x; ++q) s += sh[q];
-      phase[blockIdx.x] = s;
+    // contiguous pencils: a power of two of threads
+    for (int h = (int)blockDim.x >> 1; h > 0; h >>= 1) {
+      if ((int)threadIdx.x < h) sh[threadIdx.x] += sh[threadIdx.x + h];
+      __syncthreads();
     }
+    if (threadIdx.x == 0) phase[blockIdx.x] = sh[0];
   }
 }
 

@@ -83,3 +83,39 @@ def test_mu_with_inconsistent_dk(orc, shape):
         ctx.set_g(gs.ravel())
         ctx.sob_setup([0.5, 0.4], 0.01)
         assert np.allclose(ctx.sob_mu(), S.mu(), rtol=1e-12, atol=0)
+
+
+@pytest.mark.parametrize("c", [0.1, 0.3, 1 / 3])
+def test_long_axes_add_no_error(c):
+    # 4096 equal densities one after another in a double are off by hundreds
+    # of units of 2^-53 (N and the second moment); the sums here are exact up
+    # to a handful of roundings of their results
+    from fractions import Fraction as Fr
+    from atus2_amd import hip
+    n, dx = 4096, 0.013
+    with hip.Context((n,), [dx], [2 * np.pi / (n * dx)], 1) as ctx:
+        ctx.upload(0, np.full(n, c, np.complex128))
+        m = ctx.moments(0)
+    d, x = Fr(c * c), [Fr((j - n // 2) * dx) for j in range(n)]
+    mu = sum(x) / n
+    u = Fr(1, 2 ** 53)
+    assert abs(Fr(m["N"]) / (Fr(dx) * d * n) - 1) < 4 * u
+    assert abs(Fr(m["x2"][0]) / (sum((q - mu) ** 2 for q in x) / n) - 1) < 8 * u
+
+
+@pytest.mark.parametrize("c", [0.1, 0.7])
+def test_phase_sum_in_a_tree(c):
+    # 2^21 equal terms: 8 of a pencil, 2 tiles and 8 levels of a workgroup in
+    # a double, the rest in long double; atan2, the density, their product,
+    # the quotient by the sum and N's factor add a rounding or two each.  One
+    # after another in the workgroup and over the workgroups they are 43-48
+    # units off
+    from fractions import Fraction as Fr
+    from atus2_amd import hip
+    shape, dx = (128, 128, 128), 0.125
+    with hip.Context(shape, [dx] * 3, [2 * np.pi / 16] * 3, 1) as ctx:
+        ctx.upload(0, np.full(shape, c + 1j * c))
+        m = ctx.moments(0)
+    total = Fr(m["phase"]) * Fr(m["N"]) / Fr(dx) ** 3
+    ref = Fr(np.pi / 4) * 2 * Fr(c) ** 2 * 2 ** 21
+    assert abs(total / ref - 1) < Fr(8 + 1 + 8 + 7, 2 ** 53)
