@@ -114,17 +114,18 @@ int adam_step(atus_net* n, long long step, float lr) {
 }
 
 // floats of workspace the products of any batch up to max_batch need.  A
-// product's splits depend on its tiles, and fewer rows of tiles take more
-// splits (256 x 64 x 32768: 64 of them, 192 rows 86), so the largest batch
-// need not need the most: of the batches with the same rows of tiles it is
-// the largest
+// product's splits depend on its tiles and slices, and fewer of them can take
+// more workspace (256 rows x 64 x 32768: 64 splits, 192 rows 86), so the
+// largest batch need not need the most: of the batches with the same rows of
+// tiles and the same slices it is the largest
 size_t net_work(const int dims[5], int max_batch) {
   size_t work = 0;
-  for (int b = MLP_TILE;; b += MLP_TILE) {
+  for (int b = MLP_SLICE;; b += MLP_SLICE) {
     const int B = std::min(b, max_batch);
     for (int l = 0; l < 4; ++l) {
       const int in = dims[l], o = dims[l + 1];
       work = std::max(work, mlp_gemm_work(B, o, in));             // forward
+      work = std::max(work, mlp_gemm_work(in, o, B, true));       // dW
       if (l > 0) work = std::max(work, mlp_gemm_work(B, in, o));  // dX
     }
     if (B == max_batch) return work;

@@ -25,12 +25,13 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 // (256 x 32768 x 64 and its two transposes) stream their operands; what
 // follows them rides in their epilogues rather than in passes of its own.
 constexpr int GT = MLP_TILE;  // tile edge
-constexpr int GK = 32;        // slice along k
+constexpr int GK = MLP_SLICE; // slice along k
 constexpr int GP = GK + 8;    // LDS row pitch: 16-byte rows on distinct banks
 
 enum GemmMode {
   G_OUT = 0,    // C = act(sum + bias)
-  G_PART = 1,   // P[blockIdx.z][m][n]: partial sums of a split along k
+  G_PART = 1,   // P[blockIdx.z][m][n]: partial sums of a split along k; the
+                // column sums' partials [blockIdx.z][n] behind them
   G_MSE = 2     // d = sum + bias - T[row(m)][n]: C = 2 d / count, loss partials
 };
 
@@ -177,40 +178,48 @@ __global__ __launch_bounds__(256) void k_gemm_bf16(GemmArgs g) {
       float s = 0.f;
 #pragma unroll
       for (int q = 0; q < 4; ++q) s += red[bk ? 4 * tid + q : tid + GT * q];
-      g.e.colsum[n0 + tid] = s;
+      float* o = g.mode == G_PART ? g.C + (long long)gridDim.z * g.M * g.N + (long long)blockIdx.z * g.N : g.e.colsum;
+      o[n0 + tid] = s;
     }
   }
 }
 
-// C[m][n] = act(sum_z P[z][m][n] + bias[n]): 64 elements per workgroup, each
-// wavefront a quarter of the splits, 8 loads in flight, in a fixed order
-// (64 splits of 256 x 64 one after another in a thread took 16 us)
+// C[m][n] = act(sum_z P[z][m][n] + bias[n]), and the column sums from their
+// partials: 64 elements per workgroup, each wavefront a quarter of the
+// splits, 8 loads in flight, in a fixed order (64 splits of 256 x 64 one
+// after another in a thread took 16 us)
 __global__ __launch_bounds__(256) void k_gemm_sum(const float* __restrict__ P, int splits, int M, int N,
                                                   GemmEpilogue ep, float* __restrict__ C) {
   __shared__ float sh[4][64];
-  const long long MN = (long long)M * N;
+  const long long MN = (long long)M * N, all = MN + (ep.colsum ? N : 0);
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
   const int per = (splits + 3) / 4, z0 = w * per, z1 = min(splits, z0 + per);
-  for (long long e0 = (long long)blockIdx.x * 64; e0 < MN; e0 += (long long)gridDim.x * 64) {
+  for (long long e0 = (long long)blockIdx.x * 64; e0 < all; e0 += (long long)gridDim.x * 64) {
     const long long e = e0 + l;
+    const long long step = e < MN ? MN : N;
+    const float* p = e < MN ? P + e : P + splits * MN + (e - MN);
     float s = 0.f;
-    if (e < MN) {
+    if (e < all) {
       int z = z0;
       for (; z + 8 <= z1; z += 8) {
         float v[8];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = P[(z + i) * MN + e];
+        for (int i = 0; i < 8; ++i) v[i] = p[(z + i) * step];
 #pragma unroll
         for (int i = 0; i < 8; ++i) s += v[i];
       }
-      for (; z < z1; ++z) s += P[z * MN + e];
+      for (; z < z1; ++z) s += p[z * step];
     }
     sh[w][l] = s;
     __syncthreads();
-    if (w == 0 && e < MN) {
+    if (w == 0 && e < all) {
       s = (sh[0][l] + sh[1][l]) + (sh[2][l] + sh[3][l]);
-      if (ep.bias) s += ep.bias[e % N];
-      C[e] = gemm_act(s, ep.act, ep.X, e);
+      if (e >= MN) {
+        ep.colsum[e - MN] = s;
+      } else {
+        if (ep.bias) s += ep.bias[e % N];
+        C[e] = gemm_act(s, ep.act, ep.X, e);
+      }
     }
     __syncthreads();
   }
@@ -297,7 +306,10 @@ static unsigned ew_grid(long long n) {
 
 // Split of K: products of fewer tiles than CUs and more than 8 slices give
 // every CU a tile of at least 8 slices of its own (256 x 64 x 32768: 64
-// splits of 16 slices, 256 workgroups); shorter ones are not worth the second launch
+// splits of 16 slices, 256 workgroups); shorter ones are not worth the second
+// launch.  Weight gradients of large batches split too: unsplit, 65536 rows
+// were a chain of 2048 slices in as few workgroups as the layer has tiles
+// (WHATUS)
 static void split_plan(int M, int N, int K, int* splits, int* kchunk) {
   const long long tiles = (long long)((M + GT - 1) / GT) * ((N + GT - 1) / GT);
   const int slices = (K + GK - 1) / GK;
@@ -309,10 +321,10 @@ static void split_plan(int M, int N, int K, int* splits, int* kchunk) {
   *splits = (slices + per - 1) / per;
 }
 
-size_t mlp_gemm_work(int M, int N, int K) {
+size_t mlp_gemm_work(int M, int N, int K, bool colsum) {
   int splits, kchunk;
   split_plan(M, N, K, &splits, &kchunk);
-  return splits > 1 ? (size_t)splits * M * N : 0;
+  return splits > 1 ? (size_t)splits * (M + (colsum ? 1 : 0)) * N : 0;
 }
 
 size_t mlp_loss_parts(int M, int N) { return (size_t)((M + GT - 1) / GT) * ((N + GT - 1) / GT); }
@@ -323,12 +335,12 @@ hipError_t mlp_gemm(const float* A, long long sam, long long sak, const float* B
   if (M < 1 || N < 1 || K < 1) return hipErrorInvalidValue;
   int splits, kchunk;
   split_plan(M, N, K, &splits, &kchunk);
-  if (e.T || e.colsum) {
-    // the loss and the column sums need the whole of K in one workgroup
+  if (e.T) {
+    // the loss needs the whole of K in one workgroup
     splits = 1;
     kchunk = K;
   }
-  if (splits > 1 && (size_t)splits * M * N > work_floats) return hipErrorInvalidValue;
+  if (splits > 1 && mlp_gemm_work(M, N, K, e.colsum != nullptr) > work_floats) return hipErrorInvalidValue;
   GemmArgs g{A, sam, sak, B, sbk, sbn, splits > 1 ? work : C, M, N, K, kchunk, splits > 1 ? G_PART : e.T ? G_MSE : G_OUT,
              e};
   const long long tm = (M + GT - 1) / GT, tn = (N + GT - 1) / GT;
@@ -340,7 +352,8 @@ hipError_t mlp_gemm(const float* A, long long sam, long long sak, const float* B
     hipLaunchKernelGGL(k_gemm_bf16<false>, grid, dim3(256), 0, s, g);
   hipError_t err = hipGetLastError();
   if (err != hipSuccess || splits == 1) return err;
-  hipLaunchKernelGGL(k_gemm_sum, dim3(ew_grid((long long)M * N * 4)), dim3(256), 0, s, work, splits, M, N, e, C);
+  hipLaunchKernelGGL(k_gemm_sum, dim3(ew_grid(((long long)M + (e.colsum ? 1 : 0)) * N * 4)), dim3(256), 0, s, work, splits,
+                     M, N, e, C);
   return hipGetLastError();
 }
 

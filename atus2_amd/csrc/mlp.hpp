@@ -20,9 +20,11 @@ struct GemmEpilogue {
   float* loss = nullptr;
   float* colsum = nullptr;      // column sums of B
 };
-constexpr int MLP_TILE = 64;  // rows and columns of a product's tile
-// floats of workspace mlp_gemm needs for an M x N x K product
-size_t mlp_gemm_work(int M, int N, int K);
+constexpr int MLP_TILE = 64;   // rows and columns of a product's tile
+constexpr int MLP_SLICE = 32;  // its slices along k
+// floats of workspace mlp_gemm needs for an M x N x K product, with or without
+// column sums
+size_t mlp_gemm_work(int M, int N, int K, bool colsum = false);
 // loss partials of an M x N output
 size_t mlp_loss_parts(int M, int N);
 // C (M x N, row-major) from A B; A(m,k) = A[m*sam + k*sak], B(k,n) =

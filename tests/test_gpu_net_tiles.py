@@ -44,7 +44,8 @@ def test_forward_and_gradients(dims, batch, terms):
 @pytest.mark.parametrize("dims,max_batch,batches", [((4, 256, 256, 64, 32768), 256, (128, 191, 192)),
                                                     ((4, 256, 256, 64, 32768), 200, (101, 128, 192)),
                                                     ((4, 64, 256, 256, 32768), 65, (33, 64)),
-                                                    ((4, 16, 16, 17, 4100), 300, (1, 64, 128, 193, 256))])
+                                                    ((4, 16, 16, 17, 4100), 300, (1, 64, 128, 193, 256)),
+                                                    ((4, 65, 17, 64, 130), 2100, (511, 512, 1000, 2100))])
 def test_batches_below_the_largest(dims, max_batch, batches):
     # fewer rows of tiles are split into more parts along k: the workspace
     # holds those of every batch, not of the largest alone.  Tolerances as in
@@ -67,6 +68,30 @@ def test_batches_below_the_largest(dims, max_batch, batches):
                     assert e < 8 * 2 * u * np.linalg.norm(gref[o:o + n]), (batch, o, n, e)
             net.set_data(x, t)
             assert abs(net.train(1, batch, 1e-3)[0] / lref - 1) < 2 * 4 * 2 * u
+
+
+@pytest.mark.parametrize("dims", [(4, 16, 16, 16, 16), (3, 65, 17, 8, 33)])
+def test_gradients_of_large_batches_add_in_parts(dims):
+    # 65536 equal rows: the mean's scale is a power of two, so every addend of
+    # a gradient is 2^-16 of the one row's, exactly, and the gradients differ
+    # by what the sums round off.  A column sum adds 32 / 4 values of 8 slices
+    # in a thread, 4 threads, at most 64 splits in a wavefront and 4
+    # wavefronts; a weight 8 slices of 3 products of 32 terms, then the same.
+    # One after another the columns' threads add 16384 values each, off by
+    # 1e-4 and more.
+    from atus2_amd import hip
+    big = 65536
+    rng = np.random.default_rng(6)
+    x = rng.uniform(-1, 1, (1, dims[0])).astype(np.float32)
+    t = rng.standard_normal((1, dims[4])).astype(np.float32)
+    g = []
+    with hip.Net(dims, max_batch=big, seed=3) as net:
+        for rows in (1, big):
+            g.append(net.gradients(np.repeat(x, rows, 0), np.repeat(t, rows, 0))[1].astype(np.float64))
+    for wo, ws, bo, bn in M.layout(dims)[0]:
+        w, b = slice(wo, wo + ws[0] * ws[1]), slice(bo, bo + bn)
+        assert np.all(np.abs(g[1][b] - g[0][b]) <= (64 + 4 + 64 + 4) * 2.0 ** -24 * np.abs(g[0][b]))
+        assert np.all(np.abs(g[1][w] - g[0][w]) <= (8 * 3 * 33 + 64 + 4) * 2.0 ** -24 * np.abs(g[0][w]) + 1e-38)
 
 
 def test_training_in_chunks_equals_single_steps():
