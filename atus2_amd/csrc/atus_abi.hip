@@ -874,7 +874,6 @@ int ctx_create(atus_ctx** out, int dim, const long long n[3], const double dx[3]
     }
   }
   atus_ctx* c = new atus_ctx();
-  atus_host::staging().ref();
   c->dim = dim;
   c->ncomp = ncomp;
   c->nc_run = nc_run;
@@ -900,6 +899,8 @@ int ctx_create(atus_ctx** out, int dim, const long long n[3], const double dx[3]
     c->fs_n2 = c->n[0] / c->fs_n1;
   }
   if (hipGetDevice(&c->device) != hipSuccess) return bail(ATUS_ERR_HIP, "no HIP device");
+  c->staging = atus_host::staging(c->device);
+  if (c->staging) c->staging->ref();
   if (ensure_scratch_symbol(c->device) != ATUS_OK) {
     std::string m = g_err;
     return bail(ATUS_ERR_HIP, m);
@@ -986,7 +987,7 @@ int atus_ctx_destroy(atus_ctx* c) {
   for (hipStream_t x : c->xstream)
     if (x) (void)hipStreamDestroy(x);
   if (c->stream) (void)hipStreamDestroy(c->stream);
-  atus_host::staging().unref();
+  if (c->staging) c->staging->unref();
   delete c;
   return ATUS_OK;
 }
@@ -1011,7 +1012,8 @@ int atus_download(atus_ctx* c, int comp, double* host) {
   ATUS_TRY(check_comp(c, comp));
   if (!host) return fail(ATUS_ERR_ARG, "null host pointer");
   const double2* src = c->psi + comp * c->npts;
-  const hipError_t e = atus_host::staging().to_host(host, src, sizeof(double2) * c->npts, c->stream, c->device);
+  const hipError_t e =
+      c->staging ? c->staging->to_host(host, src, sizeof(double2) * c->npts, c->stream) : hipErrorNotReady;
   if (e != hipErrorNotReady) {
     HIP_TRY(e);
     return ATUS_OK;

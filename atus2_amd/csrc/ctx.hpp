@@ -13,6 +13,7 @@
 #include "launch.hpp"
 
 namespace atus_host {
+class Staging;
 // message of the last failure on this thread (atus_last_error)
 extern thread_local std::string g_err;
 inline int fail(int code, const std::string& msg) {
@@ -51,6 +52,7 @@ struct atus_ctx {
   double2* kinz = nullptr;  // [2 fracs][N] kinetic phases in [k1][k2] order
   double2* tbuf = nullptr;  // ncomp * npts, the transposes of full transforms
   int device = 0;
+  atus_host::Staging* staging = nullptr;  // the device's download pool, or null
   hipStream_t stream = nullptr;
   // extra streams of the slab chains (created on first use, default
   // priority), the fork event on `stream` and one join event per extra

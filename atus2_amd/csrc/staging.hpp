@@ -16,6 +16,7 @@
 #include <atomic>
 #include <cstring>
 #include <mutex>
+#include <new>
 #include <thread>
 #include <vector>
 
@@ -29,7 +30,9 @@ class Staging {
   static constexpr size_t LEAST = (size_t)1 << 20;  // shorter copies take the runtime's path
   static constexpr size_t THREADED = (size_t)8 << 20;
 
-  // the pool lives while any context does
+  explicit Staging(int device) : device_(device) {}
+
+  // the pool's memory lives while any context of its device does
   void ref() {
     std::lock_guard<std::mutex> l(m_);
     ++refs_;
@@ -43,7 +46,7 @@ class Staging {
   // `stream`; returns once dst holds them.  hipErrorNotReady: not done (a
   // short copy, another thread in the pool, no pinned memory): the caller
   // copies by itself.
-  hipError_t to_host(void* dst, const void* src, size_t bytes, hipStream_t stream, int device) {
+  hipError_t to_host(void* dst, const void* src, size_t bytes, hipStream_t stream) {
     if (bytes < LEAST) return hipErrorNotReady;
     std::unique_lock<std::mutex> l(m_, std::try_to_lock);
     if (!l.owns_lock()) return hipErrorNotReady;
@@ -51,7 +54,7 @@ class Staging {
     const size_t piece = std::min(SLOT, std::max(PIECE, (bytes / SLOTS + 4095) & ~(size_t)4095));
     const size_t n = (bytes + piece - 1) / piece;
     const int used = (int)std::min<size_t>(n, SLOTS);
-    if (!reserve(used, piece, device)) return hipErrorNotReady;
+    if (!reserve(used, piece)) return hipErrorNotReady;
     auto start = [&](size_t k, int s) {
       const size_t o = k * piece;
       hipError_t e = hipMemcpyAsync(slot_[s], (const char*)src + o, std::min(piece, bytes - o), hipMemcpyDeviceToHost,
@@ -75,7 +78,7 @@ class Staging {
       // piece k belongs to slot k % SLOTS and the thread that holds it
       std::atomic<int> first{(int)hipSuccess};
       auto work = [&](int s) {
-        hipError_t e = hipSetDevice(device);
+        hipError_t e = hipSetDevice(device_);
         for (size_t k = s; k < n && e == hipSuccess; k += SLOTS) {
           e = start(k, s);
           if (e == hipSuccess) e = finish(k, s);
@@ -101,11 +104,7 @@ class Staging {
   }
 
  private:
-  bool reserve(int used, size_t piece, int device) {
-    if (device != device_) {
-      drop();
-      device_ = device;
-    }
+  bool reserve(int used, size_t piece) {
     for (int s = 0; s < used; ++s) {
       if (!ev_[s] && hipEventCreateWithFlags(&ev_[s], hipEventDisableTiming) != hipSuccess) {
         ev_[s] = nullptr;
@@ -138,18 +137,25 @@ class Staging {
   }
 
   std::mutex m_;
+  const int device_;
   int refs_ = 0;
-  int device_ = -1;
   void* slot_[SLOTS] = {};
   size_t cap_[SLOTS] = {};
   hipEvent_t ev_[SLOTS] = {};
 };
 
-// one pool per process, never destroyed (its memory goes with the last
-// context, which may outlive static destruction)
-inline Staging& staging() {
-  static Staging* s = new Staging();
-  return *s;
+// the pool of a device (its slots and events, so that downloads from several
+// devices neither wait for each other nor take turns in one pool's slots), or
+// null; never destroyed: its memory goes with the device's last context, which
+// may outlive static destruction
+inline Staging* staging(int device) {
+  constexpr int MOST = 64;
+  static std::mutex m;
+  static Staging* pool[MOST] = {};
+  if (device < 0 || device >= MOST) return nullptr;
+  std::lock_guard<std::mutex> l(m);
+  if (!pool[device]) pool[device] = new (std::nothrow) Staging(device);
+  return pool[device];
 }
 
 }  // namespace atus_host
