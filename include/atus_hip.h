@@ -249,16 +249,21 @@ int atus_run_block_profiled(atus_ctx *ctx, const atus_step_params *sp, int Nk, d
                             double *grid);
 
 /* tuning: values per thread (8 or 16) of the FFT kernels of one kernel
- * family (ATUS_KFAM_*; the Sobolev minimiser's iteration takes 8 always).  16 halves
- * the LDS exchanges, 8 halves the registers per thread.  Defaults: 8 for
- * the strided passes and the fused V pass, and for the contiguous passes
- * and the kinetic step 16, or 8 where a run's state has fewer than 2^21
- * values. */
+ * family (ATUS_KFAM_*).  16 halves the LDS exchanges, 8 halves the registers
+ * per thread.  Defaults: 8 for the strided passes and the fused V pass, and
+ * for the contiguous passes and the kinetic step 16, or 8 where one run's
+ * state has fewer than 2^21 values.  Kernels that hold one number of values
+ * do not follow it: resident 1D blocks, the V pass of three and four
+ * components or two species, the densities along the axes, and the passes of
+ * the Sobolev minimiser along the first and the last axis (8 values; 16 on
+ * axes of 4096 points; its middle axis is a strided pass like any other).  The
+ * V pass of two components with 8 values (set or by default) is the one with
+ * a thread group per component where the state is small enough, with 16 never. */
 int atus_tune(atus_ctx *ctx, int family, int values_per_thread);
 /* tile choice of a kernel family (no reference counterpart): at most
  * `threads` threads per workgroup (64, 128, 256 or 512; 0, the default: as
- * many as the kernel allows, fewer while that leaves CUs idle), i.e. threads / (N / values_per_thread)
- * pencils per workgroup, at least one.  Fewer pencils per workgroup need
+ * many as the kernel allows, fewer while that leaves CUs idle), i.e.
+ * threads / (N / values_per_thread) pencils per workgroup, at least one.  Fewer pencils per workgroup need
  * less LDS, so more workgroups fit a CU, but strided passes then read rows
  * in shorter segments.  The results do not change. */
 int atus_tune_threads(atus_ctx *ctx, int family, int threads);
