@@ -30,14 +30,17 @@ __device__ __attribute__((noinline)) double2 sincos_large(double x) {
 // h1 + h2 + h3 with h1 of 33 bits, so n h1 is exact and x - n h1 too; t is a
 // multiple of the last bit of n h2, so what t - p rounds off is (t - r) - p
 // exactly, also where x is next to a multiple of pi/2 and r is tiny.  No
-// contraction: r has to be the difference from the rounded product.
+// contraction: r has to be the difference from the rounded product.  The
+// order of rl's terms is the one whose code costs the resident blocks nothing
+// (4096 points, 1000 steps: 9.4 ms; with the two tails added first 9.6).
 __device__ __forceinline__ double reduce_half_pi(double x, double* r, double* rl) {
 #pragma clang fp contract(off)
   const double n = rint(x * 0.6366197723675814);
   const double t = fma(-n, 1.5707963267341256, x);
   const double p = n * 6.077100506506192e-11;
-  *r = t - p;
-  *rl = ((t - *r) - p) - fma(n, 3.5215598651832e-27, fma(n, 6.077100506506192e-11, -p));
+  const double d = t - p;
+  *r = d;
+  *rl = fma(n, -3.5215598651832e-27, ((t - d) - p) - fma(n, 6.077100506506192e-11, -p));
   return n;
 }
 
@@ -53,8 +56,9 @@ __device__ __forceinline__ double reduce_half_pi(double x, double* r, double* rl
 __device__ __forceinline__ void sincos_mid(double x, double* s, double* c) {
   if (fabs(x) < 0.03125) {
     const double x2 = x * x;
-    *s = fma(x * x2, -1.0 / 6.0 + x2 * (1.0 / 120.0 + x2 * (-1.0 / 5040.0 + x2 * (1.0 / 362880.0 +
-                                                                                 x2 * (-1.0 / 39916800.0)))), x);
+    const double sx = fma(x * x2, -1.0 / 6.0 + x2 * (1.0 / 120.0 + x2 * (-1.0 / 5040.0 +
+                                                     x2 * (1.0 / 362880.0 + x2 * (-1.0 / 39916800.0)))), x);
+    *s = __builtin_copysign(sx, x);  // the sum loses the sign of zero
     *c = 1.0 + x2 * (-0.5 + x2 * (1.0 / 24.0 + x2 * (-1.0 / 720.0 + x2 * (1.0 / 40320.0 + x2 * (-1.0 / 3628800.0)))));
   } else if (fabs(x) < 1e6) {
     double r, rl;

@@ -221,3 +221,33 @@ def test_set_resident_rejects_other_values(hip):
     with hip.Context((64,), [0.5], [2 * np.pi / 32], 1) as ctx:
         with pytest.raises(hip.AtusError, match="resident"):
             hip._check(hip._lib.atus_set_resident(ctx._h, 2))
+
+
+@pytest.mark.parametrize("n,ncomp", [(1024, 1), (4096, 1), (256, 2)])
+def test_phases_beyond_a_million(n, ncomp):
+    """Resident blocks whose potential turns the phase by more than 10^6 per
+    step on part of the grid, where the V step's sine takes the library's
+    routine: against the same steps in numpy."""
+    from atus2_amd import hip
+    L, dt, nk = 20.0, 2.0 ** -13, 4
+    dx, dk = L / n, 2 * np.pi / L
+    x = (np.arange(n) - n // 2) * dx
+    k = ((np.arange(n) + n // 2) % n - n // 2) * dk
+    # powers of two, so that dt V is exact: 2^21 and 2^19
+    V = np.where(np.abs(x) > 5, 2.0 ** 34, 2.0 ** 32) * np.where(x > 0, 1.0, -1.0)
+    psis = [np.exp(-(x - 1 - c) ** 2 / 30).astype(np.complex128) for c in range(ncomp)]
+    out = [p.copy() for p in psis]
+    kin = lambda p, s: np.fft.ifft(np.fft.fft(p) * np.exp(-0.5j * s * dt * k ** 2))
+    out = [kin(p, 0.5) for p in out]
+    for m in range(nk):
+        out = [kin(p * np.exp(-1j * (dt * V)), 1.0 if m + 1 < nk else 0.5) for p in out]
+    with hip.Context((n,), [dx], [dk], ncomp) as ctx:
+        for c in range(ncomp):
+            ctx.upload(c, psis[c])
+            ctx.set_potential(c, V)
+        ctx.set_g([0.0] * ncomp ** 2)
+        ctx.set_alpha([0.5])
+        ctx.run_block(hip.STEP_FREEPROP, dt, nk, 0.0)
+        for c in range(ncomp):
+            # transforms and sines to rounding, four steps
+            assert np.linalg.norm(ctx.download(c) - out[c]) < 1e-13 * np.linalg.norm(out[c])
