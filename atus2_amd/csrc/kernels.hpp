@@ -23,8 +23,8 @@
 namespace atus {
 
 // V_NL_IF2 / V_BRAGG_DS: two species, components [NC/2, NC) are species 2
-// V_DBRAGG / V_NUM_BRAGG / V_RAMAN: three-state couplings (standalone
-// pointwise kernel only)
+// V_DBRAGG / V_NUM_BRAGG / V_RAMAN: three-state couplings (k_vcomp and the
+// standalone pointwise kernel)
 enum VKind {
   V_NONE = 0,
   V_NL = 1,

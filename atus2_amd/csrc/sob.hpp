@@ -25,7 +25,7 @@ namespace atus {
 //   k_pass      middle axis (3D) inverse (2)
 // 18.5 in 3D; the same iteration by its two filters (psi_sob, Lap psi, then
 // the gradient through the filter) takes 31.5.  At 128^3 (psi, V and the
-// spectra, 117 MiB, stay in the last-level cache) what they stream bounds
+// spectra, 112 MiB, stay in the last-level cache) what they stream bounds
 // them: an iteration takes 109 us, 5.7 TB/s, against 201 us by the filters.
 // At 32^3 their 5 launches of 3.3-6.9 us do: 26 us against 59 us for 14.
 
